@@ -5,7 +5,7 @@
 namespace cta {
 
 int64_t gemm_workspace_floats(int64_t M, int64_t N, int64_t K, int64_t Z, bool colsum) {
-  const int64_t S = splitk_factor<SplitTile>(M, N, K, Z);
+  const int64_t S = splitk_factor<WideTile>(M, N, K, Z);
   return S > 1 ? S * (Z * M * N + (colsum ? N : 0)) : 0;
 }
 
@@ -14,22 +14,18 @@ int64_t gemm_workspace_floats(int64_t M, int64_t N, int64_t K, int64_t Z, bool c
 int gemm_launch(const GemmOperand& A, const GemmOperand& B, const GemmOut& C,
                 const GemmEpilogue& ep, int64_t M, int64_t N, int64_t K, int64_t Z, int64_t zin,
                 hipStream_t st, float* workspace, int64_t workspace_floats) {
-  const int64_t S = splitk_factor<SplitTile>(M, N, K, Z);
+  const int64_t S = splitk_factor<WideTile>(M, N, K, Z);
   if (S > 1 && workspace != nullptr &&
       workspace_floats >= S * (Z * M * N + (ep.colsum ? N : 0)))
-    return gemm_launch_split(A, B, C, ep, M, N, K, Z, zin, st, workspace, workspace_floats);
-  // A product's tile never depends on its pointwise stage alone, except between the two wide
-  // tiles, which share their K-slice (hence the k pairs each MFMA sums): a fused GELU product
-  // stays bitwise equal to the plain product followed by the GELU kernel.
-  const bool n192 = N % 192 == 0;
-  if (N <= 768) {
-    if (n192 && K <= 512)
-      return gemm_launch_narrow192_short_k(A, B, C, ep, M, N, K, Z, zin, st, nullptr, 0);
-    if (n192) return gemm_launch_narrow192(A, B, C, ep, M, N, K, Z, zin, st, nullptr, 0);
-    return gemm_launch_narrow(A, B, C, ep, M, N, K, Z, zin, st, nullptr, 0);
-  }
-  if (n192 && ep.act == kActNone)
-    return gemm_launch_wide192(A, B, C, ep, M, N, K, Z, zin, st, nullptr, 0);
+    return gemm_launch_wide(A, B, C, ep, M, N, K, Z, zin, st, workspace, workspace_floats);
+  // Small outputs: 64x64 tiles while 64x128 ones would leave CUs without a workgroup (195 x 1155
+  // x 385: 20 us against 27 with 128x128 tiles).  Otherwise 64x128 for narrow outputs (16384 x
+  // 384 x 1536: 126 us, 132 with 128x128; 8192 x 768 x 3072: 248 against 262) and 128x128 for
+  // wide ones (8192 x 3072 x 768: 209 us, 239 with 64x128).  The tile never depends on the
+  // pointwise stage, and all of them sum in the same order.
+  const int64_t narrow_tiles = (M + 63) / 64 * ((N + 127) / 128) * Z;
+  if (narrow_tiles < 256) return gemm_launch_small(A, B, C, ep, M, N, K, Z, zin, st, nullptr, 0);
+  if (N <= 768) return gemm_launch_narrow(A, B, C, ep, M, N, K, Z, zin, st, nullptr, 0);
   return gemm_launch_wide(A, B, C, ep, M, N, K, Z, zin, st, nullptr, 0);
 }
 

@@ -14,17 +14,34 @@
 // The batch index z is split as (z / zin, z % zin) with a stride per level, which lets
 // the naive attention address heads inside a packed (B, T, 3C) tensor directly.
 //
-// gfx950 design: workgroup tile 128x128 of four 64x64 waves, or 64x128 of four 32x64 waves for
-// narrow outputs, each wave owning a block of v_mfma_f32_32x32x2_f32 tiles.  A and B tiles are
-// staged through LDS as [m][k] and [n][k] (k contiguous, pitch BK+4), so each MFMA operand
-// fragment is a pair of 16-byte LDS reads whatever the operand's memory order.  Operand loads
-// are dwordx4 buffer loads along whichever dimension is contiguous in memory (template mode),
-// with scalar loads for irregular strides; the epilogue stores through buffer stores.  Both
-// address a tile from scalar bases with fixed per-lane offsets and let the buffer's range check
-// zero (loads) or drop (stores) what lies outside the operand, so the K loop and the epilogue
-// carry no per-element address arithmetic or bounds tests.  Within a slice the instruction
-// order is pinned (sched_group_barrier): operand loads and LDS stores sit between the MFMAs, and
-// the next slice's fragments are read while the current slice's last MFMAs run.
+// FP32 products on the BF16 matrix pipe.  A float is the exact sum of three bfloat16 numbers
+// (8 + 8 + 8 significant bits: x0 = bf16(x), x1 = bf16(x - x0), x2 = x - x0 - x1), so
+//   a b = a0 b0 + (a0 b1 + a1 b0) + (a0 b2 + a1 b1 + a2 b0) + O(2^-26 |a b|)
+// and six v_mfma_f32_32x32x16_bf16 (32 cycles, 16 k) take the place of eight
+// v_mfma_f32_32x32x2_f32 (64 cycles, 2 k each): 192 instead of 512 matrix cycles.  The products
+// of 8-bit significands are exact and accumulate in FP32, a0 b0 apart from the other five; with
+// one rounding of the large accumulator per 16 k instead of sixteen the result is closer to the
+// exact product than the FP32 MFMA's (relative error at K = 768, N(0,1) operands: 1.6e-7 against
+// 5.0e-7; K = 8192: 5.7e-7 against 1.6e-6).
+// Sustained on all CUs, from registers, the six products reach 305 TFLOP/s of FP32 work (the
+// chip's power limit), the FP32 MFMA 154.
+// What three bfloat16 numbers cannot hold: infinities, values that round to one (above 3.39e38),
+// and the low bits of magnitudes below 2^-109.  A workgroup whose tile of sums comes out with a
+// value that is not finite, or is nonzero below 2^-100, discards it and runs the tile again with
+// FP32 MFMAs (exact_tile), so such operands give what FP32 arithmetic gives.
+//
+// gfx950 design: workgroup tile 128x128 of four 64x64 waves, 64x128 of four 32x64 or 64x64 of
+// four 32x32, two or three workgroups (waves per SIMD) on a CU.  A lane loads eight k of one row (two dwordx4
+// where k is contiguous in memory, eight coalesced dwords where the rows are), splits them
+// (11 VALU instructions per pair, in the shadow of the MFMAs) and stores one 16-byte unit per
+// part: LDS holds [part][k half][row][8 k], which is the MFMA operand order, so operand reads
+// and stores are contiguous 16-byte accesses with no bank conflict and no padding to speak of.
+// Loads and the epilogue's stores go through buffer resources: scalar bases with fixed per-lane
+// offsets, and the buffer's range check zeroes (loads) or drops (stores) what lies outside the
+// operand, so the K loop and the epilogue carry no per-element address arithmetic or bounds
+// tests.  What bounds it: 8192 x 3072 x 768 runs at 185 TFLOP/s (FP32 MFMA: 142) with the matrix
+// pipe 54% busy at 1.93 GHz, the chip's power limit (on all-zero operands the same kernel clocks
+// 2.45 GHz and takes 167 us instead of 209), so bytes moved per product cost time too.
 //
 // This header holds the kernel templates and the per-tile launcher; gemm_tiles_*.hip each
 // instantiate a few tile types (gemm_launch_<tile>), so the build compiles them in parallel, and
@@ -33,71 +50,76 @@
 
 #include "cta_common.hpp"
 #include "gemm.hpp"
+#include "split_bf16.hpp"
 
 namespace cta {
 
-enum LoadMode { kVecK = 0, kVecMN = 1, kScalar = 2 };
+// How an operand's slices are loaded: k contiguous with rows a multiple of 16 bytes apart
+// (kVecK), k contiguous with any row stride or length (kAnyK), rows contiguous (kVecMN: m of A,
+// n of B; any alignment), or any strides at all (kScalar, only ever for both operands).
+enum LoadMode { kVecK = 0, kVecMN = 1, kScalar = 2, kAnyK = 3 };
 
 namespace {
 
-// Workgroup tile BM x BN, K-slice BK, WM x WN waves; each wave owns a (BM/WM) x (BN/WN) block of
-// 32x32 MFMA tiles.  LDS rows hold one k-slice of one m (or n) index, pitch BK + 4 floats.
-template <int BM_, int BN_, int BK_, int WM_, int WN_>
+constexpr int kGemmK = 16;  // K-slice: one k step of the 32x32x16 MFMA
+
+// Workgroup tile BM x BN, WM x WN waves; each wave owns a (BM/WM) x (BN/WN) block of 32x32 MFMA
+// tiles.
+template <int BM_, int BN_, int WM_, int WN_>
 struct GemmTile {
-  static constexpr int BM = BM_, BN = BN_, BK = BK_, WM = WM_, WN = WN_;
+  static constexpr int BM = BM_, BN = BN_, WM = WM_, WN = WN_;
   static constexpr int THREADS = 64 * WM * WN;
   static constexpr int MB = BM / WM / 32;  // MFMA tiles per wave along m
   static constexpr int NB = BN / WN / 32;  // ... along n
-  static constexpr int KP = BK + 4;
-  static constexpr int LDS_FLOATS = 2 * (BM + BN) * KP;  // double buffered
-  static_assert(MB >= 1 && NB >= 1 && BK % 8 == 0, "bad GEMM tile");
+  // LDS bytes of one part of an operand's slice: two k halves of 16 bytes per row, the second
+  // 64 bytes further so that lanes writing both halves of a row use different banks.
+  static constexpr int plane(int rows) { return 2 * (rows * 16 + 64); }
+  static constexpr int A_BYTES = 3 * plane(BM), B_BYTES = 3 * plane(BN);
+  static constexpr int BUF_BYTES = A_BYTES + B_BYTES;  // double buffered
+  static_assert(MB >= 1 && NB >= 1, "bad GEMM tile");
+  static_assert(kGemmK * (BM + BN) * 4 <= 2 * BUF_BYTES, "exact_tile's slices fit");
 };
 
-// Row and k offset of float4 number f of a k-contiguous slice.  Four lanes read one row's 64
-// contiguous bytes.  With BK = 16 (LDS pitch 20 floats) a 16-byte LDS write serves 8 lanes =
-// 2 rows at once, and rows r and r+4 start 4 bank groups apart: pairing them keeps the 8
-// writes on 8 distinct bank groups.
-template <int BK>
-__device__ __forceinline__ void veck_coords(int f, int& r, int& k4) {
-  if (BK == 16) {
-    const int g = f >> 3, l = f & 7;
-    r = ((g >> 2) << 3) + (g & 3) + ((l >> 2) << 2);
-    k4 = (l & 3) * 4;
-  } else {
-    r = f / (BK / 4);
-    k4 = (f % (BK / 4)) * 4;
-  }
+// One operand's K-slice in registers: unit u of the slice is eight k (half h: k = 8h .. 8h + 7)
+// of one row; a thread holds units tid, tid + THREADS, ...  `rows` indexes m (A) or n (B); the
+// operand is row-major in (row, k) when kVecK or kAnyK, (k, row) when kVecMN.
+template <int ROWS, int THREADS>
+struct Slice {
+  static constexpr int UNITS = 2 * ROWS;
+  static constexpr int N = (UNITS + THREADS - 1) / THREADS;
+  static_assert(UNITS % 64 == 0, "whole waves hold a unit or none");
+  float v[N][8];
+};
+
+// Row and k half of unit f: in memory order, so that a wave's loads are contiguous.
+template <int MODE, int ROWS>
+__device__ __forceinline__ void unit_coords(int f, int& r, int& h) {
+  if (MODE == kVecMN) { r = f % ROWS; h = f / ROWS; }
+  else { r = f >> 1; h = f & 1; }
 }
 
-// Loads one ROWS x BK slice of an operand into registers.  `rows` indexes m (A) or n (B); the
-// operand is row-major in (row, k) when kVecK, (k, row) when kVecMN.
-//
 // Vector modes read through buffer loads: each lane's byte offset within a slice is fixed for
 // the whole K loop, and each slice only moves the resource's base and extent (scalar work), so
 // the loop carries no per-load address arithmetic.  Reads outside the resource return zero,
 // which zeroes k past the end of the K range and slices past the last one; rows past R read
-// zero (kVecK) or in-bounds values that only feed output rows/columns never stored (kVecMN).
-// On a ragged last slice a kVecK lane whose k lies past the end moves its offset out of range.
-template <int MODE, int ROWS, int BK, int THREADS>
-struct TileLoader {
-  static constexpr int LOADS = ROWS * BK / 4 / THREADS;
-  static_assert(ROWS * BK % (4 * THREADS) == 0, "tile must split evenly over the workgroup");
-  float4 v[LOADS];
-};
-
-template <int MODE, int ROWS, int BK, int THREADS>
+// zero (kVecK, kAnyK) or in-bounds values that only feed output rows/columns never stored
+// (kVecMN).  On a ragged last slice a kVecK lane whose k lies past the end moves its offset out
+// of range; kAnyK, whose end may fall inside a lane's four k, loads that slice by single dwords
+// (its whole slices are dwordx4 loads too: buffer loads need only 4-byte alignment).
+template <int MODE, int ROWS, int THREADS>
 struct LoadPlan {
-  static constexpr int LOADS = TileLoader<MODE, ROWS, BK, THREADS>::LOADS;
+  using S = Slice<ROWS, THREADS>;
+  static constexpr int N = S::N;
   const float* base;  // (row0, k0) of the tile
   int64_t s_row, s_k;
   int rows;           // valid rows from row0: min(ROWS, R - row0) (kVecK) or R - row0 (kVecMN)
   int row0, kb, R, ke;
-  int voff[LOADS];    // vector modes: byte offset of the lane's float4 within a slice
-  int kq[LOADS];      // kVecK: the float4's k within a slice
+  int voff[N];        // vector modes: byte offset of the lane's unit within a slice
+  int kq;             // kVecK, kAnyK: the unit's first k within a slice (the same for all its units)
   __device__ __forceinline__ void init(const float* b, int64_t sr, int64_t sk, int r0, int k0,
                                        int R_, int K_, int tid) {
     s_row = sr; s_k = sk; row0 = r0; kb = k0; R = R_; ke = K_;
-    if (MODE == kVecK) {
+    if (MODE == kVecK || MODE == kAnyK) {
       base = b + (int64_t)r0 * sr + k0;
       rows = min(ROWS, R_ - r0);
     } else if (MODE == kVecMN) {
@@ -106,168 +128,141 @@ struct LoadPlan {
     } else {
       base = b;
     }
+    kq = (tid & 1) * 8;
 #pragma unroll
-    for (int u = 0; u < LOADS; ++u) {
+    for (int u = 0; u < N; ++u) {
       const int f = tid + THREADS * u;
-      if (MODE == kVecMN) {
-        const int k = f % BK, r4 = (f / BK) * 4;
-        voff[u] = (int)(((int64_t)k * sk + r4) * 4);
-        kq[u] = k;
-      } else {
-        int r, k4;
-        veck_coords<BK>(f, r, k4);
-        voff[u] = (int)(((int64_t)r * sr + k4) * 4);
-        kq[u] = k4;
-      }
+      int r, h;
+      unit_coords<MODE, ROWS>(f, r, h);
+      voff[u] = MODE == kVecMN ? (int)(((int64_t)(8 * h) * sk + r) * 4)
+                               : (int)(((int64_t)r * sr + 8 * h) * 4);
+      if (f >= S::UNITS) voff[u] = (int)0x80000000;
     }
   }
-  // Slice t (k from kb + t BK) into regs.
-  __device__ __forceinline__ void load(TileLoader<MODE, ROWS, BK, THREADS>& L, int t,
-                                       int tid) const {
-    const int k0 = kb + t * BK;
-    const int klim = min(BK, ke - k0);  // <= 0 past the end: nothing in range
+  static __device__ __forceinline__ void coords(int f, int& r, int& h) {
+    unit_coords<MODE, ROWS>(f, r, h);
+  }
+  // Slice t (k from kb + t * kGemmK) into registers.
+  __device__ __forceinline__ void load(S& L, int t, int tid) const {
+    const int k0 = kb + t * kGemmK;
+    const int klim = min(kGemmK, ke - k0);  // <= 0 past the end: nothing in range
     if (MODE == kScalar) {
 #pragma unroll
-      for (int u = 0; u < LOADS; ++u) {
+      for (int u = 0; u < N; ++u) {
         const int f = tid + THREADS * u;
-        int r, k4;
-        veck_coords<BK>(f, r, k4);
-        const int gr = row0 + r, gk = k0 + k4;
-        float t4[4];
+        int r, h;
+        unit_coords<MODE, ROWS>(f, r, h);
+        const int gr = row0 + r, gk = k0 + 8 * h;
 #pragma unroll
-        for (int e = 0; e < 4; ++e)
-          t4[e] = (gr < R && gk + e < ke) ? base[(int64_t)gr * s_row + (int64_t)(gk + e) * s_k] : 0.0f;
-        L.v[u] = make_float4(t4[0], t4[1], t4[2], t4[3]);
+        for (int e = 0; e < 8; ++e)
+          L.v[u][e] = (gr < R && gk + e < ke && f < S::UNITS)
+                          ? base[(int64_t)gr * s_row + (int64_t)(gk + e) * s_k] : 0.0f;
       }
       return;
     }
     const float* bt;
     int nbytes;
-    if (MODE == kVecK) {
-      bt = base + (int64_t)t * BK;
+    if (MODE == kVecK || MODE == kAnyK) {
+      bt = base + (int64_t)t * kGemmK;
       nbytes = klim > 0 ? (int)(((int64_t)(rows - 1) * s_row + klim) * 4) : 0;
     } else {
-      bt = base + (int64_t)t * BK * s_k;
+      bt = base + (int64_t)t * kGemmK * s_k;
       nbytes = klim > 0 ? (int)(((int64_t)(klim - 1) * s_k + rows) * 4) : 0;
     }
     const __amdgpu_buffer_rsrc_t rs =
         __builtin_amdgcn_make_buffer_rsrc(const_cast<float*>(bt), (short)0, nbytes, 0x00020000);
+    if (MODE == kAnyK && klim < kGemmK) {  // uniform
 #pragma unroll
-    for (int u = 0; u < LOADS; ++u) {
-      const int vo = (MODE == kVecMN || kq[u] < klim) ? voff[u] : (int)0x80000000;
-      const u32x4 w = __builtin_amdgcn_raw_buffer_load_b128(rs, vo, 0, 0);
-      L.v[u] = make_float4(__uint_as_float(w.x), __uint_as_float(w.y), __uint_as_float(w.z),
-                           __uint_as_float(w.w));
+      for (int u = 0; u < N; ++u)
+#pragma unroll
+        for (int e = 0; e < 8; ++e)
+          L.v[u][e] = __uint_as_float(__builtin_amdgcn_raw_buffer_load_b32(
+              rs, kq + e < klim ? voff[u] + 4 * e : (int)0x80000000, 0, 0));
+      return;
+    }
+#pragma unroll
+    for (int u = 0; u < N; ++u) {
+      if (MODE == kVecK || MODE == kAnyK) {
+#pragma unroll
+        for (int q = 0; q < 2; ++q) {
+          const int vo = MODE == kAnyK || kq + 4 * q < klim ? voff[u] + 16 * q : (int)0x80000000;
+          const u32x4 w = __builtin_amdgcn_raw_buffer_load_b128(rs, vo, 0, 0);
+#pragma unroll
+          for (int e = 0; e < 4; ++e) L.v[u][4 * q + e] = __uint_as_float(w[e]);
+        }
+      } else {
+        const int kbytes = (int)(s_k * 4);
+#pragma unroll
+        for (int e = 0; e < 8; ++e)
+          L.v[u][e] = __uint_as_float(
+              __builtin_amdgcn_raw_buffer_load_b32(rs, voff[u], e * kbytes, 0));
+      }
     }
   }
 };
 
-// LDS image of a slice in regs: [row][k], pitch BK + 4.
-template <int MODE, int ROWS, int BK, int THREADS>
-__device__ __forceinline__ void store_slice(const TileLoader<MODE, ROWS, BK, THREADS>& L,
-                                            float* lds, int tid) {
-  constexpr int KP = BK + 4;
+// Splits a slice and stores its parts: LDS image [part][half][row][8 k], part p at p * PLANE.
+template <int MODE, int ROWS, int THREADS, int PLANE>
+__device__ __forceinline__ void store_slice(const Slice<ROWS, THREADS>& L, char* lds, int tid,
+                                            const SplitConsts& sc) {
+  using S = Slice<ROWS, THREADS>;
 #pragma unroll
-  for (int u = 0; u < TileLoader<MODE, ROWS, BK, THREADS>::LOADS; ++u) {
+  for (int u = 0; u < S::N; ++u) {
     const int f = tid + THREADS * u;
-    const float4 w = L.v[u];
-    if (MODE == kVecMN) {
-      const int k = f % BK, r4 = (f / BK) * 4;
-      lds[(r4 + 0) * KP + k] = w.x;
-      lds[(r4 + 1) * KP + k] = w.y;
-      lds[(r4 + 2) * KP + k] = w.z;
-      lds[(r4 + 3) * KP + k] = w.w;
-    } else {
-      int r, k4;
-      veck_coords<BK>(f, r, k4);
-      st4(lds + r * KP + k4, w);
-    }
+    if (S::UNITS % THREADS != 0 && f >= S::UNITS) continue;  // wave-uniform
+    int r, h;
+    unit_coords<MODE, ROWS>(f, r, h);
+    bf16x8 p[3];
+    split_bf16(L.v[u], p, sc);
+    char* at = lds + h * (PLANE / 2) + r * 16;
+#pragma unroll
+    for (int q = 0; q < 3; ++q) *reinterpret_cast<bf16x8*>(at + q * PLANE) = p[q];
   }
 }
 
-// One wave's operand fragments of one K-slice: per MFMA tile row (A) or column (B), KC = BK / 8
-// 16-byte chunks, each feeding four MFMAs (lane half h supplies k = 2e + h of chunk element e).
+// One wave's operand fragments of one K-slice: the three parts of each MFMA tile row (A) or
+// column (B); lane half h supplies k = 8h .. 8h + 7.
 template <class TL>
 struct Frags {
-  static constexpr int KC = TL::BK / 8;
-  float4 a[TL::MB][KC], b[TL::NB][KC];
+  bf16x8 a[TL::MB][3], b[TL::NB][3];
 };
 
-// Reads a slice's fragments from LDS: A rows [BM][KP] then B rows [BN][KP] at `as`.
 template <class TL>
-__device__ __forceinline__ void read_frags(const float* as, Frags<TL>& f, int wm, int wn,
+__device__ __forceinline__ void read_frags(const char* buf, Frags<TL>& f, int wm, int wn,
                                            int half, int col) {
-  constexpr int BM = TL::BM, BN = TL::BN, BK = TL::BK, KP = TL::KP, KC = Frags<TL>::KC;
-  const float* bs = as + BM * KP;
+  constexpr int PA = TL::plane(TL::BM), PB = TL::plane(TL::BN);
+  const char* ap = buf + half * (PA / 2) + (wm * (TL::BM / TL::WM) + col) * 16;
+  const char* bp = buf + TL::A_BYTES + half * (PB / 2) + (wn * (TL::BN / TL::WN) + col) * 16;
+  // the parts that the next slice's first products take come first
 #pragma unroll
-  for (int i = 0; i < TL::MB; ++i) {
-    const float* ap = as + (wm * (BM / TL::WM) + i * 32 + col) * KP + half * (BK / 2);
+  for (int q = 2; q >= 0; --q) {
 #pragma unroll
-    for (int c = 0; c < KC; ++c) f.a[i][c] = ld4(ap + 4 * c);
-  }
+    for (int i = 0; i < TL::MB; ++i)
+      f.a[i][q] = *reinterpret_cast<const bf16x8*>(ap + q * PA + i * 512);
 #pragma unroll
-  for (int j = 0; j < TL::NB; ++j) {
-    const float* bp = bs + (wn * (BN / TL::WN) + j * 32 + col) * KP + half * (BK / 2);
-#pragma unroll
-    for (int c = 0; c < KC; ++c) f.b[j][c] = ld4(bp + 4 * c);
-  }
-}
-
-// The MFMAs of chunks [C0, C1) of a slice, in k order for every accumulator.
-template <class TL, int C0, int C1>
-__device__ __forceinline__ void mma_chunks(const Frags<TL>& f, f32x16 (&acc)[TL::MB][TL::NB]) {
-#pragma unroll
-  for (int c = C0; c < C1; ++c)
-#pragma unroll
-    for (int e = 0; e < 4; ++e)
-#pragma unroll
-      for (int i = 0; i < TL::MB; ++i)
-#pragma unroll
-        for (int j = 0; j < TL::NB; ++j) {
-          const float4 av = f.a[i][c], bv = f.b[j][c];
-          const float a = e == 0 ? av.x : e == 1 ? av.y : e == 2 ? av.z : av.w;
-          const float b = e == 0 ? bv.x : e == 1 ? bv.y : e == 2 ? bv.z : bv.w;
-          acc[i][j] = mfma32(a, b, acc[i][j]);
-        }
-}
-
-// Instruction order of a slice's first MFMAs (sched_group_barrier masks: 0x008 MFMA,
-// 0x020 global load, 0x200 LDS store): one MFMA at a time, the next slice's global loads after
-// the first NV of them and its LDS stores, two at a time, after the middle one, so both issue
-// while the MFMA pipe is busy instead of between slices.
-template <int I, int NM, int NV, int NW>
-__device__ __forceinline__ void sched_first_part() {
-  if constexpr (I < NM) {
-    __builtin_amdgcn_sched_group_barrier(0x008, 1, 0);
-    if constexpr (I < NV) __builtin_amdgcn_sched_group_barrier(0x020, 1, 0);
-    if constexpr (I >= NM / 2 && (I - NM / 2) * 2 < NW)
-      __builtin_amdgcn_sched_group_barrier(0x200, 2, 0);
-    sched_first_part<I + 1, NM, NV, NW>();
+    for (int j = 0; j < TL::NB; ++j)
+      f.b[j][q] = *reinterpret_cast<const bf16x8*>(bp + q * PB + j * 512);
   }
 }
 
-// Instruction order of a slice's last MFMAs: all of them in a row, or with CS the column-sum
-// adds (NA VALU instructions) one after each of the first MFMAs, where the wave would otherwise
-// wait for the matrix pipe.  (The four adds in a row just before the barrier cost the kernel
-// 2-4%; one per MFMA here, 0-2%.)
-template <int N>
-__device__ __forceinline__ void sched_interleave() {
-  if constexpr (N > 0) {
-    __builtin_amdgcn_sched_group_barrier(0x008, 1, 0);
-    __builtin_amdgcn_sched_group_barrier(0x002, 1, 0);
-    sched_interleave<N - 1>();
-  }
-}
-
-template <bool CS, int NM, int NA>
-__device__ __forceinline__ void sched_second_part() {
-  if constexpr (CS) {
-    static_assert(NA <= NM, "one add per MFMA");
-    sched_interleave<NA>();
-    __builtin_amdgcn_sched_group_barrier(0x008, NM - NA, 0);
-  } else {
-    __builtin_amdgcn_sched_group_barrier(0x008, NM, 0);
-  }
+// Products [P0, P1) of the six of a slice, smallest first, in the same order for every
+// accumulator and tile type (a fused GELU product gives the bits of the plain one).  a0 b0 has
+// an accumulator of its own: the matrix pipe rounds small addends of a large accumulator
+// downward, which with one accumulator left a mean error of -4e-8 of the result's RMS at K = 768
+// (-4e-7 at 8192; column sums of such results showed it), and with two none that could be
+// measured, and a relative error of 1.6e-7 (5.7e-7) where one gives 4.2e-7 (1.4e-6).
+template <class TL, int P0, int P1>
+__device__ __forceinline__ void mma_products(const Frags<TL>& f, f32x16 (&acc)[TL::MB][TL::NB],
+                                             f32x16 (&low)[TL::MB][TL::NB]) {
+#pragma unroll
+  for (int p = P0; p < P1; ++p)
+#pragma unroll
+    for (int i = 0; i < TL::MB; ++i)
+#pragma unroll
+      for (int j = 0; j < TL::NB; ++j) {
+        f32x16& c = p == 5 ? acc[i][j] : low[i][j];
+        c = mfma_bf16(f.a[i][kSplitA[p]], f.b[j][kSplitB[p]], c);
+      }
 }
 
 // Stores a wave's block of one output tile.  RAW: the accumulators as they are (split-K
@@ -394,21 +389,71 @@ __device__ __forceinline__ void block_store(const f32x16 (&acc)[TL::MB][TL::NB],
   }
 }
 
+// The tile's sums with FP32 MFMAs, for operands that three bfloat16 parts cannot hold: the same
+// loads, FP32 slices in LDS as [k][row], one buffer.  Every thread of the workgroup calls it.
+template <class TL, class PA, class PB>
+__device__ __forceinline__ void exact_tile(const PA& pa, const PB& pb, typename PA::S& la,
+                                           typename PB::S& lb, float* smem, int nk, int tid,
+                                           int wm, int wn, int half, int col,
+                                           f32x16 (&acc)[TL::MB][TL::NB]) {
+  constexpr int BM = TL::BM, BN = TL::BN;
+#pragma unroll
+  for (int i = 0; i < TL::MB; ++i)
+#pragma unroll
+    for (int j = 0; j < TL::NB; ++j) acc[i][j] = zero16();
+  float* const as = smem;
+  float* const bs = smem + kGemmK * BM;
+  auto put = [&](const auto& plan, const auto& L, float* lds, int rows) {
+    using S = std::remove_cvref_t<decltype(L)>;
+#pragma unroll
+    for (int u = 0; u < S::N; ++u) {
+      const int f = tid + TL::THREADS * u;
+      if (f >= S::UNITS) continue;
+      int r, h;
+      plan.coords(f, r, h);
+#pragma unroll
+      for (int e = 0; e < 8; ++e) lds[(8 * h + e) * rows + r] = L.v[u][e];
+    }
+  };
+  for (int t = 0; t < nk; ++t) {
+    pa.load(la, t, tid);
+    pb.load(lb, t, tid);
+    __syncthreads();
+    put(pa, la, as, BM);
+    put(pb, lb, bs, BN);
+    __syncthreads();
+#pragma unroll
+    for (int e = 0; e < kGemmK / 2; ++e) {
+      float a[TL::MB], b[TL::NB];
+#pragma unroll
+      for (int i = 0; i < TL::MB; ++i)
+        a[i] = as[(2 * e + half) * BM + wm * (BM / TL::WM) + i * 32 + col];
+#pragma unroll
+      for (int j = 0; j < TL::NB; ++j)
+        b[j] = bs[(2 * e + half) * BN + wn * (BN / TL::WN) + j * 32 + col];
+#pragma unroll
+      for (int i = 0; i < TL::MB; ++i)
+#pragma unroll
+        for (int j = 0; j < TL::NB; ++j) acc[i][j] = mfma32(a[i], b[j], acc[i][j]);
+    }
+  }
+}
+
 // split_ws == nullptr: out = alpha * A B (+ bias, mask) written through C.
 // split_ws != nullptr: blockIdx.z = s * Z + z covers K range [s*kchunk, (s+1)*kchunk) and the raw
 // partial sum goes to split_ws[s][z][m][n] (dense); gemm_splitk_reduce finishes the epilogue.
 // CS (Z == 1, B in kVecMN mode): the workgroups of the first row of tiles also sum B's columns
 // over their K range, into ep.colsum or, split, into row s of the [S][N] block that follows
 // the partial products.
-template <class TL, int AMODE, int BMODE, int ACT, bool CS = false>
-__global__ __launch_bounds__(TL::THREADS) void gemm_kernel(GemmOperand A, GemmOperand B,
-                                                           GemmOut C, GemmEpilogue ep, int M,
-                                                           int N, int K, int zin, int Z,
-                                                           int kchunk,
-                                                           float* __restrict__ split_ws) {
-  constexpr int BM = TL::BM, BN = TL::BN, BK = TL::BK, KP = TL::KP;
+template <class TL, int AMODE, int BMODE, bool CS = false>
+__global__ __launch_bounds__(TL::THREADS, 2) void gemm_kernel(GemmOperand A, GemmOperand B,
+                                                              GemmOut C, GemmEpilogue ep, int M,
+                                                              int N, int K, int zin, int Z,
+                                                              int kchunk,
+                                                              float* __restrict__ split_ws) {
+  constexpr int BM = TL::BM, BN = TL::BN, THREADS = TL::THREADS;
   constexpr int MB = TL::MB, NB = TL::NB;
-  __shared__ __attribute__((aligned(16))) float smem[TL::LDS_FLOATS];
+  __shared__ __attribute__((aligned(16))) char smem[2 * TL::BUF_BYTES];
   const int tid = threadIdx.x;
   const int lane = tid & 63, wave = wave_index();
   const int half = lane >> 5, col = lane & 31;
@@ -440,134 +485,129 @@ __global__ __launch_bounds__(TL::THREADS) void gemm_kernel(GemmOperand A, GemmOp
   const int kb = split * kchunk;
   const int ke = min(K, kb + kchunk);
 
+  const SplitConsts sc;
   // A rows are m with (s_row, s_col) = (m, k); B "rows" are n with (n, k) = (s_col, s_row).
   // Global loads run two K-slices ahead of the MFMAs (two register sets, alternating), so a
   // slice's loads have two slices of MFMA work to arrive; LDS is double buffered.  Vector-mode
   // reads past K, or past the last slice, return zero.
-  using LA = TileLoader<AMODE, BM, BK, TL::THREADS>;
-  using LB = TileLoader<BMODE, BN, BK, TL::THREADS>;
-  LoadPlan<AMODE, BM, BK, TL::THREADS> pa;
-  LoadPlan<BMODE, BN, BK, TL::THREADS> pb;
+  using PlanA = LoadPlan<AMODE, BM, THREADS>;
+  using PlanB = LoadPlan<BMODE, BN, THREADS>;
+  constexpr int PA = TL::plane(BM), PB = TL::plane(BN);
+  PlanA pa;
+  PlanB pb;
   pa.init(Ab, A.s_row, A.s_col, m0, kb, M, ke, tid);
   pb.init(Bb, B.s_col, B.s_row, n0, kb, N, ke, tid);
-  LA la0, la1;
-  LB lb0, lb1;
-  const int nk = (ke - kb + BK - 1) / BK;
+  typename PlanA::S la0, la1;
+  typename PlanB::S lb0, lb1;
+  const int nk = (ke - kb + kGemmK - 1) / kGemmK;
   static_assert(!CS || BMODE == kVecMN, "column sums come from n-contiguous B slices");
 
-  // CS: each lane's B float4s hold the same four columns at the same k residue in every slice,
-  // so the lane sums them as the slices pass through its registers (slices past the end are
-  // zero); the lanes of one column group are combined after the loop.
-  float4 cs[CS ? LB::LOADS : 1];
-  auto add_cs = [&](const LB& lb) {
+  // CS: a lane's B unit holds the same column and k half in every slice, so the lane sums its
+  // values as the slices pass through its registers (slices past the end are zero), one sum per
+  // k of the unit: sixteen short chains a column, combined after the loop.
+  float cs[CS ? PlanB::N : 1][8];
+  auto add_cs = [&](const typename PlanB::S& lb) {
     if constexpr (CS) {
 #pragma unroll
-      for (int u = 0; u < LB::LOADS; ++u) {
-        cs[u].x += lb.v[u].x; cs[u].y += lb.v[u].y; cs[u].z += lb.v[u].z; cs[u].w += lb.v[u].w;
-      }
+      for (int u = 0; u < PlanB::N; ++u)
+#pragma unroll
+        for (int e = 0; e < 8; ++e) cs[u][e] += lb.v[u][e];
     }
   };
 #pragma unroll
-  for (int u = 0; u < (CS ? LB::LOADS : 1); ++u) cs[u] = zero4();
+  for (int u = 0; u < (CS ? PlanB::N : 1); ++u)
+#pragma unroll
+    for (int e = 0; e < 8; ++e) cs[u][e] = 0.0f;
 
-  f32x16 acc[MB][NB];
+  f32x16 acc[MB][NB], low[MB][NB];
 #pragma unroll
   for (int i = 0; i < MB; ++i)
 #pragma unroll
-    for (int j = 0; j < NB; ++j) acc[i][j] = zero16();
+    for (int j = 0; j < NB; ++j) { acc[i][j] = zero16(); low[i][j] = zero16(); }
 
   // Slice count rounded up to even: slices past the end read nothing in range, so they are
   // stored as zeros and add nothing.  The loop then has no conditional loads or stores, which
   // keeps the compiler's wait counts exact (a load issued two slices ahead is not waited for
   // until its LDS store).
   const int nk2 = (nk + 1) & ~1;
+  char* const buf0 = smem;
+  char* const buf1 = smem + TL::BUF_BYTES;
   pa.load(la0, 0, tid);
   pb.load(lb0, 0, tid);
   pa.load(la1, 1, tid);
   pb.load(lb1, 1, tid);
-  store_slice(la0, smem, tid);
-  store_slice(lb0, smem + BM * KP, tid);
+  store_slice<AMODE, BM, THREADS, PA>(la0, buf0, tid, sc);
+  store_slice<BMODE, BN, THREADS, PB>(lb0, buf0 + TL::A_BYTES, tid, sc);
   add_cs(lb0);
   __syncthreads();
 
   // Each slice's MFMAs run in two parts around the barrier that publishes the next slice.  The
-  // first part carries the next-but-one slice's global loads and the next slice's LDS stores;
-  // right after the barrier the wave issues the next slice's fragment reads, which complete
-  // under the second part, so no wave waits on LDS latency before its MFMAs.  A buffer is
-  // rewritten only after the barrier that follows every wave's reads of it (the barrier waits
-  // for outstanding LDS reads).
-  constexpr int KC = Frags<TL>::KC;
-  static_assert(KC % 2 == 0, "a slice splits into two halves of chunks");
-  constexpr int NM1 = MB * NB * 4 * (KC / 2);  // MFMAs per part
-  constexpr int NVM = LA::LOADS + LB::LOADS;
-  constexpr int NDW = LA::LOADS * (AMODE == kVecMN ? 4 : 1) + LB::LOADS * (BMODE == kVecMN ? 4 : 1);
-  constexpr int NDR = (MB + NB) * KC;
-  float* const buf0 = smem;
-  float* const buf1 = smem + (BM + BN) * KP;
+  // first part (the three smallest products) carries the next-but-one slice's global loads and
+  // the next slice's split and LDS stores; right after the barrier the wave issues the next
+  // slice's fragment reads, which complete under the second part, so no wave waits on LDS
+  // latency before its MFMAs.  A buffer is rewritten only after the barrier that follows every
+  // wave's reads of it (the barrier waits for outstanding LDS reads).
   Frags<TL> f0, f1;
   read_frags<TL>(buf0, f0, wm, wn, half, col);
+  auto slice = [&](Frags<TL>& cur, Frags<TL>& nxt, typename PlanA::S& la_far,
+                   typename PlanB::S& lb_far, const typename PlanA::S& la_next,
+                   const typename PlanB::S& lb_next, char* nbuf, int t_far) {
+    pa.load(la_far, t_far, tid);
+    pb.load(lb_far, t_far, tid);
+    mma_products<TL, 0, 3>(cur, acc, low);
+    store_slice<AMODE, BM, THREADS, PA>(la_next, nbuf, tid, sc);
+    store_slice<BMODE, BN, THREADS, PB>(lb_next, nbuf + TL::A_BYTES, tid, sc);
+    add_cs(lb_next);
+    __syncthreads();
+    read_frags<TL>(nbuf, nxt, wm, wn, half, col);
+    mma_products<TL, 3, 6>(cur, acc, low);
+  };
   for (int t = 0; t < nk2; t += 2) {
     // slice t in f0; slices t+2 (set 0) and t+1 (set 1, stored below) in flight
-    pa.load(la0, t + 2, tid);
-    pb.load(lb0, t + 2, tid);
-    mma_chunks<TL, 0, KC / 2>(f0, acc);
-    store_slice(la1, buf1, tid);
-    store_slice(lb1, buf1 + BM * KP, tid);
-    sched_first_part<0, NM1, NVM, NDW>();
-    __builtin_amdgcn_sched_barrier(0);
-    __syncthreads();
-    __builtin_amdgcn_sched_barrier(0);
-    read_frags<TL>(buf1, f1, wm, wn, half, col);
-    mma_chunks<TL, KC / 2, KC>(f0, acc);
-    add_cs(lb1);
-    __builtin_amdgcn_sched_group_barrier(0x100, NDR, 0);  // LDS reads first
-    sched_second_part<CS, NM1, 4 * LB::LOADS>();
-    __builtin_amdgcn_sched_barrier(0);
-    // slice t+1 in f1
-    pa.load(la1, t + 3, tid);
-    pb.load(lb1, t + 3, tid);
-    mma_chunks<TL, 0, KC / 2>(f1, acc);
-    store_slice(la0, buf0, tid);
-    store_slice(lb0, buf0 + BM * KP, tid);
-    sched_first_part<0, NM1, NVM, NDW>();
-    __builtin_amdgcn_sched_barrier(0);
-    __syncthreads();
-    __builtin_amdgcn_sched_barrier(0);
-    read_frags<TL>(buf0, f0, wm, wn, half, col);
-    mma_chunks<TL, KC / 2, KC>(f1, acc);
-    add_cs(lb0);
-    __builtin_amdgcn_sched_group_barrier(0x100, NDR, 0);
-    sched_second_part<CS, NM1, 4 * LB::LOADS>();
-    __builtin_amdgcn_sched_barrier(0);
+    slice(f0, f1, la0, lb0, la1, lb1, buf1, t + 2);
+    slice(f1, f0, la1, lb1, la0, lb0, buf0, t + 3);
   }
 
+  // Sums that the split cannot vouch for (see the top): the whole workgroup runs the tile again.
+  bool odd = false;
+#pragma unroll
+  for (int i = 0; i < MB; ++i)
+#pragma unroll
+    for (int j = 0; j < NB; ++j) {
+      acc[i][j] += low[i][j];
+      odd |= split_suspect(acc[i][j]);
+    }
+  if (__syncthreads_or(odd))
+    exact_tile<TL>(pa, pb, la0, lb0, reinterpret_cast<float*>(smem), nk, tid, wm, wn, half, col,
+                   acc);
+
   if constexpr (CS) {
-    if (m0 == 0) {
-      // Lanes f with the same f / BK share a column group (BK consecutive lanes of one wave).
+    if (m0 == 0) {  // workgroup-uniform
+      // Units f and f + BN hold the two k halves of column f.
+      float* const half1 = reinterpret_cast<float*>(smem);
+      auto unit_sum = [&](int u) {
+        return ((cs[u][0] + cs[u][1]) + (cs[u][2] + cs[u][3])) +
+               ((cs[u][4] + cs[u][5]) + (cs[u][6] + cs[u][7]));
+      };
+      __syncthreads();  // every wave is done with the slices
+#pragma unroll
+      for (int u = 0; u < PlanB::N; ++u) {
+        const int f = tid + THREADS * u;
+        if (f >= BN && f < 2 * BN) half1[f - BN] = unit_sum(u);
+      }
+      __syncthreads();
       float* out = split_ws ? split_ws + (int64_t)gridDim.z * M * N + (int64_t)split * N
                             : ep.colsum;
 #pragma unroll
-      for (int u = 0; u < LB::LOADS; ++u) {
-        float4 v = cs[u];
-#pragma unroll
-        for (int off = 1; off < BK; off <<= 1) {
-          v.x += __shfl_xor(v.x, off);
-          v.y += __shfl_xor(v.y, off);
-          v.z += __shfl_xor(v.z, off);
-          v.w += __shfl_xor(v.w, off);
-        }
-        const int f = tid + TL::THREADS * u;
-        const int n = n0 + (f / BK) * 4;
-        if (f % BK == 0 && n < N) {  // N % 4 == 0: the whole group is in range
-          out[n] = v.x; out[n + 1] = v.y; out[n + 2] = v.z; out[n + 3] = v.w;
-        }
+      for (int u = 0; u < PlanB::N; ++u) {
+        const int f = tid + THREADS * u;
+        if (f < BN && n0 + f < N) out[n0 + f] = unit_sum(u) + half1[f];
       }
     }
   }
 
   const int mw = m0 + wm * (BM / TL::WM), nw = n0 + wn * (BN / TL::WN);
   if (mw >= M || nw >= N) return;
-  // The block's byte extent must fit the 32-bit buffer offsets; the launcher checks it.
   if (split_ws != nullptr) {
     float* Pz = split_ws + ((int64_t)split * Z + z) * M * N;
     block_store<TL, kActNone, true, false>(acc, Pz, nullptr, N, ep, M, N, mw, nw, half, col);
@@ -575,10 +615,24 @@ __global__ __launch_bounds__(TL::THREADS) void gemm_kernel(GemmOperand A, GemmOp
   }
   float* Cz = C.p + zo * C.s_outer + zi * C.s_inner;
   float* Xz = ep.aux ? ep.aux + zo * C.s_outer + zi * C.s_inner : nullptr;
-  if (ep.causal_mask)
-    block_store<TL, ACT, false, true>(acc, Cz, Xz, C.s_row, ep, M, N, mw, nw, half, col);
-  else
-    block_store<TL, ACT, false, false>(acc, Cz, Xz, C.s_row, ep, M, N, mw, nw, half, col);
+  // The pointwise stage is a scalar branch here, outside the K loop: one kernel per tile and
+  // operand order instead of one per stage.
+  auto store = [&]<int ACT, bool MASK>() {
+    block_store<TL, ACT, false, MASK>(acc, Cz, Xz, C.s_row, ep, M, N, mw, nw, half, col);
+  };
+  if constexpr (CS) {
+    store.template operator()<kActNone, false>();
+    return;
+  }
+  if (ep.causal_mask) store.template operator()<kActNone, true>();
+  else if (ep.act == kActNone) store.template operator()<kActNone, false>();
+  else if (ep.act == kActGelu) store.template operator()<kActGelu, false>();
+  else if (ep.act == kActGeluGrad) store.template operator()<kActGeluGrad, false>();
+  else if (ep.act == kActGeluTanh) store.template operator()<kActGeluTanh, false>();
+  else if (ep.act == kActGeluTanhGrad) store.template operator()<kActGeluTanhGrad, false>();
+  else if (ep.act == kActGeluDeriv) store.template operator()<kActGeluDeriv, false>();
+  else if (ep.act == kActGeluTanhDeriv) store.template operator()<kActGeluTanhDeriv, false>();
+  else store.template operator()<kActMulAux, false>();
 }
 
 // Fixed-order sum of the split-K partials plus the epilogue of gemm_kernel; with ep.colsum also
@@ -618,81 +672,83 @@ __global__ __launch_bounds__(256) void gemm_splitk_reduce(const float* __restric
   }
 }
 
-bool vec_ok(const GemmOperand& op, bool contig_is_col) {
-  // dwordx4 loads along the contiguous dimension need 16-byte aligned rows.
-  const int64_t s_other = contig_is_col ? op.s_row : op.s_col;
-  return aligned16(op.p) && s_other % 4 == 0 && op.s_outer % 4 == 0 && op.s_inner % 4 == 0;
-}
-
 // Load mode of an operand.  A: (s_row, s_col) = (m, k); B: (k, n).  `rows` is M for A and N for
-// B.  The vector modes also need the contiguous extent to be a multiple of 4 (a float4 lies
-// wholly inside or outside the operand) and at least 4.
+// B.
 int pick_mode(const GemmOperand& op, bool is_a, int64_t rows, int64_t K) {
   const int64_t s_k = is_a ? op.s_col : op.s_row;
   const int64_t s_mn = is_a ? op.s_row : op.s_col;
-  // The buffer loads address a slice with 32-bit byte offsets and rely on rows (kVecK) or
+  // The buffer loads address a slice with 32-bit byte offsets and rely on rows (kVecK, kAnyK) or
   // k rows (kVecMN) not overlapping, so that reads past the valid range fall outside it.
   constexpr int64_t kMaxBytes = (int64_t)1 << 31;
-  if (s_k == 1 && K % 4 == 0 && K >= 4 && vec_ok(op, is_a) && s_mn >= K &&
-      (255 * s_mn + 64) * 4 < kMaxBytes)
-    return kVecK;
-  if (s_mn == 1 && rows % 4 == 0 && rows >= 4 && vec_ok(op, !is_a) && s_k >= rows &&
+  if (s_k == 1 && K >= 1 && s_mn >= K && (255 * s_mn + 64) * 4 < kMaxBytes) {
+    // dwordx4 loads of a ragged end need it to fall between float4s
+    const bool quads = K % 4 == 0 && aligned16(op.p) && s_mn % 4 == 0 && op.s_outer % 4 == 0 &&
+                       op.s_inner % 4 == 0;
+    return quads ? kVecK : kAnyK;
+  }
+  if (s_mn == 1 && rows >= 1 && s_k >= rows &&
       (63 * s_k + std::max<int64_t>(rows, 256)) * 4 < kMaxBytes)
     return kVecMN;
   return kScalar;
 }
 
-template <class TL, int AM, int ACT, bool CS>
+template <class TL, int AM, bool CS>
 void dispatch_b(int bm, dim3 grid, hipStream_t st, const GemmOperand& A, const GemmOperand& B,
                 const GemmOut& C, const GemmEpilogue& ep, int M, int N, int K, int zin, int Z,
                 int kchunk, float* ws) {
   const dim3 block(TL::THREADS);
   if constexpr (CS) {  // the launcher has checked bm == kVecMN
-    hipLaunchKernelGGL((gemm_kernel<TL, AM, kVecMN, ACT, true>), grid, block, 0, st, A, B, C, ep,
-                       M, N, K, zin, Z, kchunk, ws);
+    hipLaunchKernelGGL((gemm_kernel<TL, AM, kVecMN, true>), grid, block, 0, st, A, B, C, ep, M, N,
+                       K, zin, Z, kchunk, ws);
     return;
   }
   if (bm == kVecK)
-    hipLaunchKernelGGL((gemm_kernel<TL, AM, kVecK, ACT>), grid, block, 0, st, A, B, C, ep, M, N,
-                       K, zin, Z, kchunk, ws);
-  else if (bm == kVecMN)
-    hipLaunchKernelGGL((gemm_kernel<TL, AM, kVecMN, ACT>), grid, block, 0, st, A, B, C, ep, M, N,
-                       K, zin, Z, kchunk, ws);
+    hipLaunchKernelGGL((gemm_kernel<TL, AM, kVecK>), grid, block, 0, st, A, B, C, ep, M, N, K,
+                       zin, Z, kchunk, ws);
+  else if (bm == kAnyK)
+    hipLaunchKernelGGL((gemm_kernel<TL, AM, kAnyK>), grid, block, 0, st, A, B, C, ep, M, N, K,
+                       zin, Z, kchunk, ws);
   else
-    hipLaunchKernelGGL((gemm_kernel<TL, AM, kScalar, ACT>), grid, block, 0, st, A, B, C, ep, M,
-                       N, K, zin, Z, kchunk, ws);
+    hipLaunchKernelGGL((gemm_kernel<TL, AM, kVecMN>), grid, block, 0, st, A, B, C, ep, M, N, K,
+                       zin, Z, kchunk, ws);
 }
 
-template <class TL, int ACT, bool CS = false>
+template <class TL, bool CS = false>
 void dispatch_a(int am, int bm, dim3 grid, hipStream_t st, const GemmOperand& A,
                 const GemmOperand& B, const GemmOut& C, const GemmEpilogue& ep, int M, int N,
                 int K, int zin, int Z, int kchunk, float* ws) {
+  // kScalar loads any layout: one kernel of it serves wherever either operand needs it
+  if (!CS && (am == kScalar || bm == kScalar)) {
+    hipLaunchKernelGGL((gemm_kernel<TL, kScalar, kScalar>), grid, dim3(TL::THREADS), 0, st, A, B,
+                       C, ep, M, N, K, zin, Z, kchunk, ws);
+    return;
+  }
   if (am == kVecK)
-    dispatch_b<TL, kVecK, ACT, CS>(bm, grid, st, A, B, C, ep, M, N, K, zin, Z, kchunk, ws);
+    dispatch_b<TL, kVecK, CS>(bm, grid, st, A, B, C, ep, M, N, K, zin, Z, kchunk, ws);
+  else if (am == kAnyK)
+    dispatch_b<TL, kAnyK, CS>(bm, grid, st, A, B, C, ep, M, N, K, zin, Z, kchunk, ws);
   else if (am == kVecMN)
-    dispatch_b<TL, kVecMN, ACT, CS>(bm, grid, st, A, B, C, ep, M, N, K, zin, Z, kchunk, ws);
-  else
-    dispatch_b<TL, kScalar, ACT, CS>(bm, grid, st, A, B, C, ep, M, N, K, zin, Z, kchunk, ws);
+    dispatch_b<TL, kVecMN, CS>(bm, grid, st, A, B, C, ep, M, N, K, zin, Z, kchunk, ws);
+  else if constexpr (CS)
+    dispatch_b<TL, kScalar, true>(bm, grid, st, A, B, C, ep, M, N, K, zin, Z, kchunk, ws);
 }
 
 // K splits for a GEMM whose output tiles alone cannot fill the 256 CUs (1 = no split).  The
 // busiest CU runs ceil(tiles S / 256) workgroups of ceil(K / S) each, and the split adds a
 // round trip of S partial outputs through HBM; S in [1, 32] (at least 256 of K per split)
-// minimises the sum.  Costs are in seconds at an MFMA rate of ~0.4 TFLOP/s per CU and
-// ~5 TB/s of HBM.  E.g. the 768 x 3072 x 8192 weight gradient: 144 tiles, S = 7 (1008
-// workgroups, 98% of the CUs' time busy) where a plain "~512 workgroups" rule gives S = 4
-// (576 workgroups, three rounds for 2.25 rounds of work); the 384 x 384 x 16384 one: 9 tiles,
-// S = 28 (252 workgroups; capped at 16 it left 112 CUs idle and ran 27% slower).
+// minimises the sum.  Costs are in seconds at ~1.2 TFLOP/s per CU and ~5 TB/s of HBM.  E.g. the
+// 768 x 3072 x 8192 weight gradient: 144 tiles, S = 5 (234 us + 17 us of reduction; S = 7, which
+// the FP32 MFMA's 0.4 TFLOP/s gave, 235 + 20).
 template <class TL>
 int64_t splitk_factor(int64_t M, int64_t N, int64_t K, int64_t Z) {
   const int64_t tiles = ((M + TL::BM - 1) / TL::BM) * ((N + TL::BN - 1) / TL::BN) * Z;
   if (tiles >= 256 || K < 1024) return 1;
-  constexpr double kCuFlops = 0.4e12, kHbmBytes = 5e12;
+  constexpr double kCuFlops = 1.2e12, kHbmBytes = 5e12;
   const double tile_flop_per_k = 2.0 * TL::BM * TL::BN;
   int64_t best = 1;
   double best_cost = 0.0;
   for (int64_t s = 1; s <= 32 && (s == 1 || K / s >= 256); ++s) {
-    const int64_t kchunk = ((K + s - 1) / s + TL::BK - 1) / TL::BK * TL::BK;
+    const int64_t kchunk = ((K + s - 1) / s + kGemmK - 1) / kGemmK * kGemmK;
     const int64_t rounds = (tiles * s + 255) / 256;
     const double cost = (double)rounds * kchunk * tile_flop_per_k / kCuFlops +
                         (s > 1 ? 8.0 * s * M * N * Z / kHbmBytes : 0.0);
@@ -701,8 +757,7 @@ int64_t splitk_factor(int64_t M, int64_t N, int64_t K, int64_t Z) {
   return best;
 }
 
-// ACTS = false: a tile instantiated without the pointwise stages (ep.act must be kActNone).
-template <class TL, bool ACTS = true>
+template <class TL>
 int gemm_launch_tile(const GemmOperand& A, const GemmOperand& B, const GemmOut& C,
                      const GemmEpilogue& ep, int64_t M, int64_t N, int64_t K, int64_t Z,
                      int64_t zin, hipStream_t st, float* workspace, int64_t workspace_floats) {
@@ -713,7 +768,7 @@ int gemm_launch_tile(const GemmOperand& A, const GemmOperand& B, const GemmOut& 
   const int64_t cs_floats = ep.colsum ? N : 0;  // per split
   if (S > 1 && (workspace == nullptr || workspace_floats < S * (Z * M * N + cs_floats))) S = 1;
   const int64_t kchunk =
-      S > 1 ? ((K + S - 1) / S + TL::BK - 1) / TL::BK * TL::BK : std::max<int64_t>(K, 1);
+      S > 1 ? ((K + S - 1) / S + kGemmK - 1) / kGemmK * kGemmK : std::max<int64_t>(K, 1);
   const int64_t ntiles = ((N + TL::BN - 1) / TL::BN) * ((M + TL::BM - 1) / TL::BM);
   if (ntiles * Z > INT32_MAX - kNumXcds || Z * S > 65535)
     return fail(CTA_ERR_INVALID_ARGUMENT, "GEMM grid too large");
@@ -724,36 +779,16 @@ int gemm_launch_tile(const GemmOperand& A, const GemmOperand& B, const GemmOut& 
   float* ws = S > 1 ? workspace : nullptr;
   const int am = pick_mode(A, true, M, K);
   const int bm = pick_mode(B, false, N, K);
-  // Split-K partials are stored raw; the reduction applies the epilogue's pointwise stage.
-  const int act = S > 1 ? kActNone : ep.act;
   const int iM = (int)M, iN = (int)N, iK = (int)K, izin = (int)zin, iZ = (int)Z, ikc = (int)kchunk;
   if (ep.colsum) {
     if (Z != 1 || bm != kVecMN || ep.act != kActNone || ep.causal_mask)
       return fail(CTA_ERR_INVALID_ARGUMENT,
                   "GEMM column sums need one batch, an n-contiguous B and no pointwise stage");
-    dispatch_a<TL, kActNone, true>(am, bm, grid, st, A, B, C, ep, iM, iN, iK, izin, iZ, ikc, ws);
-  } else if constexpr (!ACTS) {
-    if (act != kActNone) return fail(CTA_ERR_INVALID_ARGUMENT, "GEMM tile without pointwise stages");
-    dispatch_a<TL, kActNone>(am, bm, grid, st, A, B, C, ep, iM, iN, iK, izin, iZ, ikc, ws);
+    dispatch_a<TL, true>(am, bm, grid, st, A, B, C, ep, iM, iN, iK, izin, iZ, ikc, ws);
   } else {
-    if (act == kActGelu)
-      dispatch_a<TL, kActGelu>(am, bm, grid, st, A, B, C, ep, iM, iN, iK, izin, iZ, ikc, ws);
-    else if (act == kActGeluGrad)
-      dispatch_a<TL, kActGeluGrad>(am, bm, grid, st, A, B, C, ep, iM, iN, iK, izin, iZ, ikc, ws);
-    else if (act == kActGeluTanh)
-      dispatch_a<TL, kActGeluTanh>(am, bm, grid, st, A, B, C, ep, iM, iN, iK, izin, iZ, ikc, ws);
-    else if (act == kActGeluTanhGrad)
-      dispatch_a<TL, kActGeluTanhGrad>(am, bm, grid, st, A, B, C, ep, iM, iN, iK, izin, iZ, ikc,
-                                       ws);
-    else if (act == kActGeluDeriv)
-      dispatch_a<TL, kActGeluDeriv>(am, bm, grid, st, A, B, C, ep, iM, iN, iK, izin, iZ, ikc, ws);
-    else if (act == kActGeluTanhDeriv)
-      dispatch_a<TL, kActGeluTanhDeriv>(am, bm, grid, st, A, B, C, ep, iM, iN, iK, izin, iZ, ikc,
-                                        ws);
-    else if (act == kActMulAux)
-      dispatch_a<TL, kActMulAux>(am, bm, grid, st, A, B, C, ep, iM, iN, iK, izin, iZ, ikc, ws);
-    else
-      dispatch_a<TL, kActNone>(am, bm, grid, st, A, B, C, ep, iM, iN, iK, izin, iZ, ikc, ws);
+    if (ep.causal_mask && ep.act != kActNone)
+      return fail(CTA_ERR_INVALID_ARGUMENT, "GEMM with both a mask and a pointwise stage");
+    dispatch_a<TL>(am, bm, grid, st, A, B, C, ep, iM, iN, iK, izin, iZ, ikc, ws);
   }
   if (S > 1) {
     const int64_t total = Z * M * N + cs_floats;
@@ -764,40 +799,21 @@ int gemm_launch_tile(const GemmOperand& A, const GemmOperand& B, const GemmOut& 
   return check_launch("gemm");
 }
 
-// Tile choice, from measured sweeps of the config-4 and small-GPT shapes on an MI355X:
-// narrow outputs (N <= 768) run best with a 64x128 tile of four 32x64 waves and K-slices of 32,
-// wider ones with a 128x128 tile of four 64x64 waves, and shapes split along K with a 128x128
-// tile of eight 32x64 waves.  When N is a multiple of 192 the same shapes with 192 columns
-// (waves of 32x96 or 64x96) measured 0-8% faster (cold, A/B in one process): 64x192 with
-// K-slices of 16 for K <= 512 and of 32 beyond, and, without a pointwise stage, 128x192 with
-// K-slices of 16 for N > 768 (with the GELU stages it was slower in the GPT step).
-using SplitTile = GemmTile<128, 128, 16, 4, 2>;
-using NarrowTile = GemmTile<64, 128, 32, 2, 2>;
-using Narrow192Tile = GemmTile<64, 192, 32, 2, 2>;
-using Narrow192ShortKTile = GemmTile<64, 192, 16, 2, 2>;
-using WideTile = GemmTile<128, 128, 16, 2, 2>;
-using Wide192Tile = GemmTile<128, 192, 16, 2, 2>;
+using WideTile = GemmTile<128, 128, 2, 2>;
+using NarrowTile = GemmTile<64, 128, 2, 2>;
+using SmallTile = GemmTile<64, 64, 2, 2>;
 
 }  // namespace
 
 // One launcher per tile type (defined in gemm_tiles_*.hip): gemm_launch_tile of that tile.
-int gemm_launch_split(const GemmOperand& A, const GemmOperand& B, const GemmOut& C,
-                      const GemmEpilogue& ep, int64_t M, int64_t N, int64_t K, int64_t Z,
-                      int64_t zin, hipStream_t st, float* workspace, int64_t workspace_floats);
-int gemm_launch_narrow(const GemmOperand& A, const GemmOperand& B, const GemmOut& C,
-                       const GemmEpilogue& ep, int64_t M, int64_t N, int64_t K, int64_t Z,
-                       int64_t zin, hipStream_t st, float* workspace, int64_t workspace_floats);
-int gemm_launch_narrow192(const GemmOperand& A, const GemmOperand& B, const GemmOut& C,
-                          const GemmEpilogue& ep, int64_t M, int64_t N, int64_t K, int64_t Z,
-                          int64_t zin, hipStream_t st, float* workspace, int64_t workspace_floats);
-int gemm_launch_narrow192_short_k(const GemmOperand& A, const GemmOperand& B, const GemmOut& C,
-                                  const GemmEpilogue& ep, int64_t M, int64_t N, int64_t K, int64_t Z,
-                                  int64_t zin, hipStream_t st, float* workspace, int64_t workspace_floats);
 int gemm_launch_wide(const GemmOperand& A, const GemmOperand& B, const GemmOut& C,
                      const GemmEpilogue& ep, int64_t M, int64_t N, int64_t K, int64_t Z,
                      int64_t zin, hipStream_t st, float* workspace, int64_t workspace_floats);
-int gemm_launch_wide192(const GemmOperand& A, const GemmOperand& B, const GemmOut& C,
-                        const GemmEpilogue& ep, int64_t M, int64_t N, int64_t K, int64_t Z,
-                        int64_t zin, hipStream_t st, float* workspace, int64_t workspace_floats);
+int gemm_launch_narrow(const GemmOperand& A, const GemmOperand& B, const GemmOut& C,
+                       const GemmEpilogue& ep, int64_t M, int64_t N, int64_t K, int64_t Z,
+                       int64_t zin, hipStream_t st, float* workspace, int64_t workspace_floats);
+int gemm_launch_small(const GemmOperand& A, const GemmOperand& B, const GemmOut& C,
+                      const GemmEpilogue& ep, int64_t M, int64_t N, int64_t K, int64_t Z,
+                      int64_t zin, hipStream_t st, float* workspace, int64_t workspace_floats);
 
 }  // namespace cta
