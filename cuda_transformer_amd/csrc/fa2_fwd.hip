@@ -6,14 +6,25 @@
 // gfx950:
 //
 //  * A workgroup owns BM = 128 query rows (4 waves x 32 rows; 64 rows of 2 waves for short
-//    causal heads).  K/V tiles of BN rows are
-//    staged global -> registers -> LDS, double buffered, one barrier per tile.
-//  * Each wave computes S^T = K Q^T with v_mfma_f32_32x32x2_f32.  In the MFMA output layout
-//    lane l then holds 16 scores of query row (l % 32) — one row per lane — so the row max
-//    needs one in-lane max over 16 registers and one exchange with the other wave half.
-//  * O^T = V^T P^T reuses the score registers directly as the B operand: the K index of the
-//    second MFMA is permuted to match the output layout of the first, and V is read from LDS
-//    in the same permuted order.  P never leaves registers.
+//    causal heads).  Both products run on the BF16 matrix pipe with FP32 operands split into
+//    three bfloat16 parts, six products of parts each (gemm_kernel.hpp): 1536 matrix cycles per
+//    32x32 score tile at hs 64 where the FP32 MFMA takes 4096.  At B4 H32 N4096 D64 causal the
+//    forward takes 1.51 ms (182 TFLOP/s), 2.18 on FP32 MFMAs, with an error against float64 of
+//    2.1e-7 instead of 5.0e-7.  What bounds it: the VALU work beside the MFMAs (the softmax and
+//    the splits of P, K and V, about 900 of each tile's cycles) at two waves per SIMD, and the
+//    chip's power limit.
+//  * K/V stages of 32 rows go global -> registers -> split -> LDS, double buffered, one barrier
+//    per stage; the LDS image is in MFMA operand order (K by rows, V transposed), so operand
+//    reads are contiguous 16-byte accesses.  Q's parts stay in registers.
+//  * Each wave computes S^T = K Q^T.  In the MFMA output layout lane l then holds 16 scores of
+//    query row (l % 32) - one row per lane - so the row max needs one in-lane max over 16
+//    registers and one exchange with the other wave half.
+//  * O^T = V^T P^T takes the score registers, split in place, as the B operand: registers
+//    8s .. 8s + 7 are step s's eight keys of this lane's half, and V's image holds its keys in
+//    that order.  P never leaves registers.
+//  * A pass whose sums are not finite, or nonzero below 2^-100, is run again on FP32 MFMAs by
+//    the whole workgroup, so infinities, NaN and the ends of FP32's range give what FP32
+//    arithmetic gives.
 //  * Exponentials use exp2 with log2(e) folded into the scale; L is exported in natural log.
 //  * Lazy rescaling: the running max m used as the exponent offset only moves when some row
 //    of the wave sees a tile max more than 2^8 above it (a wave-uniform vote).  Otherwise the
@@ -28,6 +39,7 @@
 //    fill the resident slots each XCD instead takes single tiles of its heads longest first
 //    (lpt_heads).
 #include "cta_common.hpp"
+#include "split_bf16.hpp"
 
 namespace cta {
 namespace {
@@ -36,11 +48,50 @@ struct RowStrides {
   int64_t b, h, t;  // element strides of the batch, head and time axes (d-stride is 1)
 };
 
+// BN key rows per stage; MINW waves per SIMD that the registers are held to.
 template <int HS>
 struct FwdTile;
 template <> struct FwdTile<32> { static constexpr int BN = 32; static constexpr int MINW = 2; };
 template <> struct FwdTile<64> { static constexpr int BN = 32; static constexpr int MINW = 2; };
 template <> struct FwdTile<128> { static constexpr int BN = 32; static constexpr int MINW = 1; };
+
+// One online-softmax step of a wave's 32x32 score tile (lane: 16 scores of its query row): the
+// mask, the lazily moved offset m and P = 2^{(S - m) c} in place of S.  `rescale(alpha)` scales
+// the output accumulators when the offset moves.
+template <bool CAUSAL, class F>
+__device__ __forceinline__ void softmax_step(f32x16& sacc, int jj0, int i0, int my_i, int T,
+                                             int half, float scale_log2, float rescale_gap,
+                                             float& m_run, float& l_run, F&& rescale) {
+  const bool need_mask = (CAUSAL && jj0 + 31 > i0) || (jj0 + 32 > T);
+  if (need_mask) {
+#pragma unroll
+    for (int r = 0; r < 16; ++r) {
+      const int j = jj0 + mfma_row(r, half);
+      if ((CAUSAL && j > my_i) || j >= T) sacc[r] = -INFINITY;
+    }
+  }
+  float mt = sacc[0];
+#pragma unroll
+  for (int r = 1; r < 16; ++r) mt = fmaxf(mt, sacc[r]);
+  mt = max_halves(mt);
+  // rescale_gap = 8 / scale_log2: a tile max within 2^8 of m keeps the old offset.
+  // The first tile always rescales (m_run = -inf), with alpha = 0 on zero accumulators.
+  if (__any(mt > m_run + rescale_gap)) {
+    const float m_new = fmaxf(m_run, mt);
+    const float alpha = fast_exp2((m_run - m_new) * scale_log2);
+    l_run *= alpha;
+    rescale(alpha);
+    m_run = m_new;
+  }
+  float psum = 0.0f;
+#pragma unroll
+  for (int r = 0; r < 16; ++r) {
+    const float p = fast_exp2((sacc[r] - m_run) * scale_log2);
+    sacc[r] = p;
+    psum += p;
+  }
+  l_run += psum;
+}
 
 // NSPLIT > 1: each work item (query-tile pair, or tile) is run by NSPLIT workgroups, parts 0 ..
 // NSPLIT - 1, each over a contiguous share of the item's K/V stages (in the item's stage order,
@@ -57,15 +108,21 @@ __global__ __launch_bounds__(64 * WAVES, FwdTile<HS>::MINW) void fa2_fwd_kernel(
   constexpr int BN = FwdTile<HS>::BN;
   constexpr int THREADS = 64 * WAVES;
   constexpr int BM = 32 * WAVES;  // query rows per workgroup, 32 per wave
-  constexpr int H2 = HS / 2;    // d values per lane half
-  constexpr int KP = HS + 4;    // LDS pitch (floats) of a K row: conflict-free 16-byte row reads
-  constexpr int VP = HS + 8;    // LDS pitch of a V row: the two wave halves read rows 4 apart
-  constexpr int KTILE = BN * KP;
-  constexpr int VTILE = BN * VP;
-  constexpr int F4_ROW = HS / 4;
-  constexpr int LOADS = BN * F4_ROW / THREADS;
-  static_assert(BN * F4_ROW % THREADS == 0, "tile must split evenly over the workgroup");
-  __shared__ __attribute__((aligned(16))) float smem[2 * (KTILE + VTILE)];
+  static_assert(BN == 32, "a stage is one score tile");
+  // LDS image of a stage, in units of eight values of one bfloat16 part (16 bytes): K unit
+  // (d8, key) = d 8 d8 .. 8 d8 + 7 of a key row, at d8 * 32 + (key ^ (d8 & 7)) (the swizzle
+  // spreads a row's units, written by neighbouring lanes, over the banks); V unit (d, sh) = the
+  // eight keys that half sh & 1 of the PV product's step sh >> 1 takes, at (d/32, sh, d % 32).
+  // Either way one MFMA operand read is 64 consecutive units, part by part.
+  constexpr int PART = BN * HS * 2;   // bytes of one part of a K (or V) stage
+  constexpr int STAGE = 6 * PART;
+  constexpr int KUNITS = BN * HS / 8; // units a part: of K, and of V
+  constexpr int NU = (KUNITS + THREADS - 1) / THREADS;
+  static_assert(KUNITS % 64 == 0, "whole waves hold a unit or none");
+  constexpr int KP = HS + 4, VP = HS + 8;  // row pitches of the FP32 stage (exact_pass)
+  static_assert(BN * (KP + VP) * 4 <= 2 * STAGE, "the FP32 stage fits");
+  __shared__ __attribute__((aligned(16))) char smem[2 * STAGE];
+  const SplitConsts sc;
 
   const int tid = threadIdx.x;
   const int lane = tid & 63, wave = wave_index();
@@ -118,22 +175,24 @@ __global__ __launch_bounds__(64 * WAVES, FwdTile<HS>::MINW) void fa2_fwd_kernel(
   const int i0 = qt * BM + wave * 32;  // first query row of this wave
   const int my_i = i0 + col;           // query row owned by this lane
 
-  float qf[H2];
-  if (my_i < T) {
-    const float* qp = Qb + (int64_t)my_i * sq.t + half * H2;
+  // Q parts of this lane's row, the B operands of the score product: step s, d 16s + 8 half + j.
+  bf16x8 qp[HS / 16][3];
 #pragma unroll
-    for (int c = 0; c < H2 / 4; ++c) {
-      float4 x = ld4(qp + 4 * c);
-      qf[4 * c + 0] = x.x; qf[4 * c + 1] = x.y; qf[4 * c + 2] = x.z; qf[4 * c + 3] = x.w;
+  for (int st = 0; st < HS / 16; ++st) {
+    float x[8];
+    const float* q8 = Qb + (int64_t)my_i * sq.t + 16 * st + 8 * half;
+#pragma unroll
+    for (int c = 0; c < 2; ++c) {
+      const float4 v = my_i < T ? ld4(q8 + 4 * c) : zero4();
+      x[4 * c] = v.x; x[4 * c + 1] = v.y; x[4 * c + 2] = v.z; x[4 * c + 3] = v.w;
     }
-  } else {
-#pragma unroll
-    for (int c = 0; c < H2; ++c) qf[c] = 0.0f;
+    split_bf16(x, qp[st], sc);
   }
 
-  f32x16 oacc[HS / 32];
+  // O: the products of the first parts and the smaller ones apart (see gemm_kernel.hpp)
+  f32x16 oacc[HS / 32], olow[HS / 32];
 #pragma unroll
-  for (int d = 0; d < HS / 32; ++d) oacc[d] = zero16();
+  for (int d = 0; d < HS / 32; ++d) { oacc[d] = zero16(); olow[d] = zero16(); }
   float m_run = -INFINITY;  // exponent offset of row my_i (raw q.k units), lazily updated
   float l_run = 0.0f;       // this lane's partial row sum (its half of the columns)
   // The exponents are (S - m) s log2(e): the subtraction comes first, so the row maximum gets
@@ -147,7 +206,7 @@ __global__ __launch_bounds__(64 * WAVES, FwdTile<HS>::MINW) void fa2_fwd_kernel(
   const int i_end = SPLIT ? min(max(g1 - pos, 0), n_stages) : n_stages;
   pos += n_stages;
 
-  float4 kst[LOADS], vst[LOADS];
+  float kst[NU][8], vst[NU][8];
   // K/V rows of a stage through buffer resources over its valid rows (scalar base and extent;
   // the lanes' offsets are the same every stage): rows past T read as zero.
   auto gload = [&](int stage) {
@@ -155,23 +214,42 @@ __global__ __launch_bounds__(64 * WAVES, FwdTile<HS>::MINW) void fa2_fwd_kernel(
     const int rows = min(BN, T - j0);
     const __amdgpu_buffer_rsrc_t rk = rows_rsrc(Kb + (int64_t)j0 * sk.t, rows, sk.t, HS);
     const __amdgpu_buffer_rsrc_t rv = rows_rsrc(Vb + (int64_t)j0 * sv.t, rows, sv.t, HS);
+    const int st = (int)sv.t * 4;
 #pragma unroll
-    for (int u = 0; u < LOADS; ++u) {
+    for (int u = 0; u < NU; ++u) {
       const int f = tid + THREADS * u;
-      const int r = f / F4_ROW, c4 = f % F4_ROW;
-      kst[u] = ld4_buffer(rk, (r * (int)sk.t + 4 * c4) * 4);
-      vst[u] = ld4_buffer(rv, (r * (int)sv.t + 4 * c4) * 4);
+      if (KUNITS % THREADS != 0 && f >= KUNITS) continue;  // wave-uniform
+      const int key = f / (HS / 8), d8 = f % (HS / 8);
+      const int vk = (key * (int)sk.t + 8 * d8) * 4;
+      const float4 x = ld4_buffer(rk, vk), y = ld4_buffer(rk, vk + 16);
+      kst[u][0] = x.x; kst[u][1] = x.y; kst[u][2] = x.z; kst[u][3] = x.w;
+      kst[u][4] = y.x; kst[u][5] = y.y; kst[u][6] = y.z; kst[u][7] = y.w;
+      const int d = f % HS, sh = f / HS;
+      const int vv = (16 * (sh >> 1) + 4 * (sh & 1)) * st + 4 * d;
+#pragma unroll
+      for (int j = 0; j < 8; ++j)
+        vst[u][j] = __uint_as_float(__builtin_amdgcn_raw_buffer_load_b32(
+            rv, vv, (8 * (j >> 2) + (j & 3)) * st, 0));
     }
   };
   auto lstore = [&](int buf) {
-    float* ks = smem + buf * (KTILE + VTILE);
-    float* vs = ks + KTILE;
+    char* ks = smem + buf * STAGE;
+    char* vs = ks + 3 * PART;
 #pragma unroll
-    for (int u = 0; u < LOADS; ++u) {
+    for (int u = 0; u < NU; ++u) {
       const int f = tid + THREADS * u;
-      const int r = f / F4_ROW, c4 = f % F4_ROW;
-      st4(ks + r * KP + 4 * c4, kst[u]);
-      st4(vs + r * VP + 4 * c4, vst[u]);
+      if (KUNITS % THREADS != 0 && f >= KUNITS) continue;
+      const int key = f / (HS / 8), d8 = f % (HS / 8);
+      const int d = f % HS, sh = f / HS;
+      bf16x8 p[3];
+      split_bf16(kst[u], p, sc);
+#pragma unroll
+      for (int q = 0; q < 3; ++q)
+        *reinterpret_cast<bf16x8*>(ks + q * PART + (d8 * 32 + (key ^ (d8 & 7))) * 16) = p[q];
+      split_bf16(vst[u], p, sc);
+#pragma unroll
+      for (int q = 0; q < 3; ++q)
+        *reinterpret_cast<bf16x8*>(vs + q * PART + ((d >> 5) * 128 + sh * 32 + (d & 31)) * 16) = p[q];
     }
   };
 
@@ -193,70 +271,110 @@ __global__ __launch_bounds__(64 * WAVES, FwdTile<HS>::MINW) void fa2_fwd_kernel(
     const int s = stage_at(i);
     const int buf = (i - i_begin) & 1;
     if (i + 1 < i_end) gload(stage_at(i + 1));
-    const float* ks = smem + buf * (KTILE + VTILE);
-    const float* vs = ks + KTILE;
-
+    const char* ks = smem + buf * STAGE;
+    const char* vs = ks + 3 * PART;
+    const int jj0 = s * BN;
+    if (!(CAUSAL && jj0 > i0 + 31)) {  // else the tile lies above this wave's diagonal
+      // S^T tile: lane holds q_{my_i} . k_{jj0 + R(r, half)}.  Two chains, even and odd steps.
+      f32x16 sacc = zero16(), sodd = zero16();
 #pragma unroll
-    for (int sub = 0; sub < BN / 32; ++sub) {
-      const int jj0 = s * BN + sub * 32;
-      if (jj0 >= T) continue;                      // ragged tail: nothing left in this stage
-      if (CAUSAL && jj0 > i0 + 31) continue;       // tile entirely above this wave's diagonal
-
-      // S^T tile: sacc[r] = q_{my_i} . k_{jj0 + R(r, half)}
-      f32x16 sacc = zero16();
-      const float* krow = ks + (sub * 32 + col) * KP + half * H2;
+      for (int st = 0; st < HS / 16; st += 2) {
+        bf16x8 ka[2][3];
 #pragma unroll
-      for (int c = 0; c < H2 / 4; ++c) {
-        const float4 kv = ld4(krow + 4 * c);
-        sacc = mfma32(kv.x, qf[4 * c + 0], sacc);
-        sacc = mfma32(kv.y, qf[4 * c + 1], sacc);
-        sacc = mfma32(kv.z, qf[4 * c + 2], sacc);
-        sacc = mfma32(kv.w, qf[4 * c + 3], sacc);
-      }
-
-      const bool need_mask = (CAUSAL && jj0 + 31 > i0) || (jj0 + 32 > T);
-      if (need_mask) {
+        for (int o = 0; o < 2; ++o) {
+          const int d8 = 2 * (st + o) + half;
+          const char* at = ks + (d8 * 32 + (col ^ (d8 & 7))) * 16;
 #pragma unroll
-        for (int r = 0; r < 16; ++r) {
-          const int j = jj0 + mfma_row(r, half);
-          if ((CAUSAL && j > my_i) || j >= T) sacc[r] = -INFINITY;
+          for (int q = 2; q >= 0; --q) ka[o][q] = *reinterpret_cast<const bf16x8*>(at + q * PART);
+        }
+#pragma unroll
+        for (int p = 0; p < 6; ++p) {
+          sacc = mfma_bf16(ka[0][kSplitA[p]], qp[st][kSplitB[p]], sacc);
+          sodd = mfma_bf16(ka[1][kSplitA[p]], qp[st + 1][kSplitB[p]], sodd);
         }
       }
-
-      float mt = sacc[0];
+      sacc += sodd;
+      softmax_step<CAUSAL>(sacc, jj0, i0, my_i, T, half, scale_log2, rescale_gap, m_run, l_run,
+                           [&](float alpha) {
 #pragma unroll
-      for (int r = 1; r < 16; ++r) mt = fmaxf(mt, sacc[r]);
-      mt = max_halves(mt);
-      // rescale_gap = 8 / scale_log2: a tile max within 2^8 of m keeps the old offset.
-      // The first tile always rescales (m_run = -inf), with alpha = 0 on zero accumulators.
-      if (__any(mt > m_run + rescale_gap)) {
-        const float m_new = fmaxf(m_run, mt);
-        const float alpha = fast_exp2((m_run - m_new) * scale_log2);
-        l_run *= alpha;
+                             for (int d = 0; d < HS / 32; ++d) { oacc[d] *= alpha; olow[d] *= alpha; }
+                           });
+      // O^T += V^T P^T, two steps of 16 keys
 #pragma unroll
-        for (int d = 0; d < HS / 32; ++d) oacc[d] *= alpha;
-        m_run = m_new;
-      }
-      float psum = 0.0f;
+      for (int st = 0; st < 2; ++st) {
+        float x[8];
 #pragma unroll
-      for (int r = 0; r < 16; ++r) {
-        const float p = fast_exp2((sacc[r] - m_run) * scale_log2);
-        sacc[r] = p;
-        psum += p;
-      }
-      l_run += psum;
-
+        for (int e = 0; e < 8; ++e) x[e] = sacc[8 * st + e];
+        bf16x8 pp[3], va[HS / 32][3];
 #pragma unroll
-      for (int d = 0; d < HS / 32; ++d) {
+        for (int d = 0; d < HS / 32; ++d)
 #pragma unroll
-        for (int kk = 0; kk < 16; ++kk) {
-          const float a = vs[(sub * 32 + mfma_row(kk, half)) * VP + d * 32 + col];
-          oacc[d] = mfma32(a, sacc[kk], oacc[d]);
-        }
+          for (int q = 2; q >= 0; --q)
+            va[d][q] = *reinterpret_cast<const bf16x8*>(
+                vs + q * PART + (d * 128 + (2 * st + half) * 32 + col) * 16);
+        split_bf16(x, pp, sc);
+#pragma unroll
+        for (int p = 0; p < 6; ++p)
+#pragma unroll
+          for (int d = 0; d < HS / 32; ++d) {
+            f32x16& c = p == 5 ? oacc[d] : olow[d];
+            c = mfma_bf16(va[d][kSplitA[p]], pp[kSplitB[p]], c);
+          }
       }
     }
 
     if (i + 1 < i_end) lstore(buf ^ 1);
+    __syncthreads();
+  }
+
+  // Sums that the split cannot vouch for (not finite, or nonzero below 2^-100; see
+  // split_bf16.hpp): the workgroup runs the pass again on FP32 MFMAs.
+  bool odd = !(l_run < INFINITY);
+#pragma unroll
+  for (int d = 0; d < HS / 32; ++d) {
+    oacc[d] += olow[d];
+    odd |= split_suspect(oacc[d]);
+  }
+  if (__syncthreads_or(odd)) {
+    float* const ks = reinterpret_cast<float*>(smem);
+    float* const vs = ks + BN * KP;
+    m_run = -INFINITY;
+    l_run = 0.0f;
+#pragma unroll
+    for (int d = 0; d < HS / 32; ++d) oacc[d] = zero16();
+    for (int i = i_begin; i < i_end; ++i) {
+      const int jj0 = stage_at(i) * BN;
+      __syncthreads();
+      for (int f = tid; f < BN * HS / 4; f += THREADS) {
+        const int r = f / (HS / 4), c4 = f % (HS / 4) * 4;
+        const int64_t j = jj0 + r;
+        st4(ks + r * KP + c4, j < T ? ld4(Kb + j * sk.t + c4) : zero4());
+        st4(vs + r * VP + c4, j < T ? ld4(Vb + j * sv.t + c4) : zero4());
+      }
+      __syncthreads();
+      if (CAUSAL && jj0 > i0 + 31) continue;
+      f32x16 sacc = zero16();
+      const float* q = Qb + (int64_t)min(my_i, T - 1) * sq.t + half * (HS / 2);
+      const float* krow = ks + col * KP + half * (HS / 2);
+#pragma unroll 2
+      for (int c = 0; c < HS / 8; ++c) {
+        const float4 x = ld4(q + 4 * c), y = ld4(krow + 4 * c);
+        sacc = mfma32(y.x, x.x, sacc);
+        sacc = mfma32(y.y, x.y, sacc);
+        sacc = mfma32(y.z, x.z, sacc);
+        sacc = mfma32(y.w, x.w, sacc);
+      }
+      softmax_step<CAUSAL>(sacc, jj0, i0, my_i, T, half, scale_log2, rescale_gap, m_run, l_run,
+                           [&](float alpha) {
+#pragma unroll
+                             for (int d = 0; d < HS / 32; ++d) oacc[d] *= alpha;
+                           });
+#pragma unroll
+      for (int d = 0; d < HS / 32; ++d)
+#pragma unroll
+        for (int kk = 0; kk < 16; ++kk)
+          oacc[d] = mfma32(vs[mfma_row(kk, half) * VP + d * 32 + col], sacc[kk], oacc[d]);
+    }
     __syncthreads();
   }
 
@@ -351,12 +469,11 @@ __global__ __launch_bounds__(256) void fa2_fwd_merge_kernel(float* __restrict__ 
 }
 
 // The forward splits each work item's K/V stages over NSPLIT workgroups when its grid would hold
-// fewer than two waves per SIMD (1024 SIMDs): enough parts to fill the waves per SIMD its
-// registers and LDS allow (three at hs 32 / 64, two at hs 128), each part keeping at least
-// kSplitMinStages stages; the merge pass is the cost.  A/B in one process against the unsplit
-// forward: B4 H4 N4096 causal 0.3306 -> 0.3042 ms with two parts (+8.7%), B2 H4 N4096
-// non-causal +7.3%; at T = 256 (B64 H6, 8 stages per row) two parts were 30% slower, the merge
-// outweighing the work, hence the minimum.
+// fewer than two waves per SIMD (1024 SIMDs): up to three parts at hs 32 / 64 and two at hs 128,
+// each keeping at least kSplitMinStages stages; the merge pass is the cost.  B4 H4 N4096 causal
+// takes 235 us in three parts (two: 227; on FP32 MFMAs, which held three waves per SIMD, 298 in
+// three); callers size their workspace by this rule, so it stays.  At T = 256 (B64 H6, 8 stages
+// per row) two parts were 30% slower, the merge outweighing the work, hence the minimum.
 constexpr int kSimds = 1024;
 constexpr int kSplitMinStages = 16;
 
@@ -372,7 +489,7 @@ int fwd_nsplit(int T, int BH) {
   const int n_qtiles = (T + 32 * waves - 1) / (32 * waves);
   const int64_t w = (int64_t)(CAUSAL ? (n_qtiles + 1) / 2 : n_qtiles) * BH * waves;
   if (w >= 2 * kSimds) return 1;
-  const int occ = HS == 128 ? 2 : 3;  // waves per SIMD the unsplit kernel can hold
+  const int occ = HS == 128 ? 2 : 3;
   int n = (int)std::min<int64_t>(occ, (occ * kSimds + w - 1) / w);
   n = std::min(n, T / FwdTile<HS>::BN / kSplitMinStages);
   return n >= 2 ? n : 1;
@@ -410,11 +527,9 @@ void launch_fwd(const float* q, const float* k, const float* v, float* o, float*
       split.template operator()<2>();
       return;
     }
-    // Slots counted at three waves per SIMD for hs 32 / 64 (the four-wave kernel's 160 VGPRs
-    // hold three; the two-wave one's 186 hold two, but measured, its longest-first tiles win at
-    // B64 H6 T256, 1.5 rounds of them at two waves, +9%, and lose at B8 H32 T512, 2 rounds, -3%,
-    // which the three-wave count separates).
-    const int lpt = CAUSAL ? lpt_heads(BH, n_qtiles, WAVES, HS == 128 ? 1 : 3) : 0;
+    // Slots counted at the two waves per SIMD the kernel holds (one at hs 128): B64 H6 T256
+    // takes 43.7 us, 45.3 with three counted.
+    const int lpt = CAUSAL ? lpt_heads(BH, n_qtiles, WAVES, HS == 128 ? 1 : 2) : 0;
     hipLaunchKernelGGL((fa2_fwd_kernel<HS, CAUSAL, WAVES>),
                        dim3(lpt > 0 ? (unsigned)(BH * n_qtiles) : xcd_grid(items)),
                        dim3(64 * WAVES), 0, stream, q, k, v, o, l, nh, T, BH, n_qtiles, sq, sk,
