@@ -122,7 +122,6 @@ __global__ __launch_bounds__(64 * WAVES, FwdTile<HS>::MINW) void fa2_fwd_kernel(
   constexpr int KP = HS + 4, VP = HS + 8;  // row pitches of the FP32 stage (exact_pass)
   static_assert(BN * (KP + VP) * 4 <= 2 * STAGE, "the FP32 stage fits");
   __shared__ __attribute__((aligned(16))) char smem[2 * STAGE];
-  const SplitConsts sc;
 
   const int tid = threadIdx.x;
   const int lane = tid & 63, wave = wave_index();
@@ -186,7 +185,7 @@ __global__ __launch_bounds__(64 * WAVES, FwdTile<HS>::MINW) void fa2_fwd_kernel(
       const float4 v = my_i < T ? ld4(q8 + 4 * c) : zero4();
       x[4 * c] = v.x; x[4 * c + 1] = v.y; x[4 * c + 2] = v.z; x[4 * c + 3] = v.w;
     }
-    split_bf16(x, qp[st], sc);
+    split_bf16(x, qp[st]);
   }
 
   // O: the products of the first parts and the smaller ones apart (see gemm_kernel.hpp)
@@ -242,11 +241,11 @@ __global__ __launch_bounds__(64 * WAVES, FwdTile<HS>::MINW) void fa2_fwd_kernel(
       const int key = f / (HS / 8), d8 = f % (HS / 8);
       const int d = f % HS, sh = f / HS;
       bf16x8 p[3];
-      split_bf16(kst[u], p, sc);
+      split_bf16(kst[u], p);
 #pragma unroll
       for (int q = 0; q < 3; ++q)
         *reinterpret_cast<bf16x8*>(ks + q * PART + (d8 * 32 + (key ^ (d8 & 7))) * 16) = p[q];
-      split_bf16(vst[u], p, sc);
+      split_bf16(vst[u], p);
 #pragma unroll
       for (int q = 0; q < 3; ++q)
         *reinterpret_cast<bf16x8*>(vs + q * PART + ((d >> 5) * 128 + sh * 32 + (d & 31)) * 16) = p[q];
@@ -312,7 +311,7 @@ __global__ __launch_bounds__(64 * WAVES, FwdTile<HS>::MINW) void fa2_fwd_kernel(
           for (int q = 2; q >= 0; --q)
             va[d][q] = *reinterpret_cast<const bf16x8*>(
                 vs + q * PART + (d * 128 + (2 * st + half) * 32 + col) * 16);
-        split_bf16(x, pp, sc);
+        split_bf16(x, pp);
 #pragma unroll
         for (int p = 0; p < 6; ++p)
 #pragma unroll

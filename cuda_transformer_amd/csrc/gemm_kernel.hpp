@@ -33,7 +33,7 @@
 // gfx950 design: workgroup tile 128x128 of four 64x64 waves, 64x128 of four 32x64 or 64x64 of
 // four 32x32, two or three workgroups (waves per SIMD) on a CU.  A lane loads eight k of one row (two dwordx4
 // where k is contiguous in memory, eight coalesced dwords where the rows are), splits them
-// (11 VALU instructions per pair, in the shadow of the MFMAs) and stores one 16-byte unit per
+// (11 VALU instructions per pair, beside the MFMAs) and stores one 16-byte unit per
 // part: LDS holds [part][k half][row][8 k], which is the MFMA operand order, so operand reads
 // and stores are contiguous 16-byte accesses with no bank conflict and no padding to speak of.
 // Loads and the epilogue's stores go through buffer resources: scalar bases with fixed per-lane
@@ -203,8 +203,7 @@ struct LoadPlan {
 
 // Splits a slice and stores its parts: LDS image [part][half][row][8 k], part p at p * PLANE.
 template <int MODE, int ROWS, int THREADS, int PLANE>
-__device__ __forceinline__ void store_slice(const Slice<ROWS, THREADS>& L, char* lds, int tid,
-                                            const SplitConsts& sc) {
+__device__ __forceinline__ void store_slice(const Slice<ROWS, THREADS>& L, char* lds, int tid) {
   using S = Slice<ROWS, THREADS>;
 #pragma unroll
   for (int u = 0; u < S::N; ++u) {
@@ -213,7 +212,7 @@ __device__ __forceinline__ void store_slice(const Slice<ROWS, THREADS>& L, char*
     int r, h;
     unit_coords<MODE, ROWS>(f, r, h);
     bf16x8 p[3];
-    split_bf16(L.v[u], p, sc);
+    split_bf16(L.v[u], p);
     char* at = lds + h * (PLANE / 2) + r * 16;
 #pragma unroll
     for (int q = 0; q < 3; ++q) *reinterpret_cast<bf16x8*>(at + q * PLANE) = p[q];
@@ -485,7 +484,6 @@ __global__ __launch_bounds__(TL::THREADS, 2) void gemm_kernel(GemmOperand A, Gem
   const int kb = split * kchunk;
   const int ke = min(K, kb + kchunk);
 
-  const SplitConsts sc;
   // A rows are m with (s_row, s_col) = (m, k); B "rows" are n with (n, k) = (s_col, s_row).
   // Global loads run two K-slices ahead of the MFMAs (two register sets, alternating), so a
   // slice's loads have two slices of MFMA work to arrive; LDS is double buffered.  Vector-mode
@@ -536,8 +534,8 @@ __global__ __launch_bounds__(TL::THREADS, 2) void gemm_kernel(GemmOperand A, Gem
   pb.load(lb0, 0, tid);
   pa.load(la1, 1, tid);
   pb.load(lb1, 1, tid);
-  store_slice<AMODE, BM, THREADS, PA>(la0, buf0, tid, sc);
-  store_slice<BMODE, BN, THREADS, PB>(lb0, buf0 + TL::A_BYTES, tid, sc);
+  store_slice<AMODE, BM, THREADS, PA>(la0, buf0, tid);
+  store_slice<BMODE, BN, THREADS, PB>(lb0, buf0 + TL::A_BYTES, tid);
   add_cs(lb0);
   __syncthreads();
 
@@ -555,8 +553,8 @@ __global__ __launch_bounds__(TL::THREADS, 2) void gemm_kernel(GemmOperand A, Gem
     pa.load(la_far, t_far, tid);
     pb.load(lb_far, t_far, tid);
     mma_products<TL, 0, 3>(cur, acc, low);
-    store_slice<AMODE, BM, THREADS, PA>(la_next, nbuf, tid, sc);
-    store_slice<BMODE, BN, THREADS, PB>(lb_next, nbuf + TL::A_BYTES, tid, sc);
+    store_slice<AMODE, BM, THREADS, PA>(la_next, nbuf, tid);
+    store_slice<BMODE, BN, THREADS, PB>(lb_next, nbuf + TL::A_BYTES, tid);
     add_cs(lb_next);
     __syncthreads();
     read_frags<TL>(nbuf, nxt, wm, wn, half, col);

@@ -17,22 +17,7 @@ __device__ __forceinline__ f32x16 mfma_bf16(bf16x8 a, bf16x8 b, f32x16 c) {
 constexpr int kSplitA[6] = {0, 1, 2, 0, 1, 0};
 constexpr int kSplitB[6] = {2, 1, 0, 1, 0, 0};
 
-// x - the low (high) half of a packed bfloat16 pair, exact where the half is x rounded:
-// v_dot2_f32_bf16 with the constant (-1, 0) or (0, -1), one instruction where unpacking the half
-// and subtracting take two.  The constants are kept in scalar registers: the compiler would
-// encode (-1, 0) as the inline constant -1.0, which this instruction reads as a float's bits.
 typedef __bf16 bf16x2 __attribute__((ext_vector_type(2)));
-struct SplitConsts {
-  uint32_t lo, hi;
-  __device__ __forceinline__ SplitConsts() {
-    asm("s_mov_b32 %0, 0xbf80" : "=s"(lo));
-    asm("s_mov_b32 %0, 0xbf800000" : "=s"(hi));
-  }
-};
-__device__ __forceinline__ float minus_half(uint32_t pair, uint32_t half, float x) {
-  return __builtin_amdgcn_fdot2_f32_bf16(__builtin_bit_cast(bf16x2, pair),
-                                         __builtin_bit_cast(bf16x2, half), x, false);
-}
 __device__ __forceinline__ uint32_t pack_bf16(float lo, float hi) {
   typedef float f32x2 __attribute__((ext_vector_type(2)));
   const f32x2 v = {lo, hi};
@@ -40,18 +25,22 @@ __device__ __forceinline__ uint32_t pack_bf16(float lo, float hi) {
 }
 
 // x = p[0] + p[1] + p[2], each part rounded to nearest.  The differences are exact; the last
-// part holds what is left in at most 8 bits (above 2^-109).  Seven instructions a pair.
-__device__ __forceinline__ void split_bf16(const float (&x)[8], bf16x8 (&p)[3],
-                                           const SplitConsts& c) {
+// part holds what is left in at most 8 bits (above 2^-109).  Eleven instructions a pair, all of
+// which run beside the MFMAs (up to five for each 32-cycle MFMA).  v_dot2_f32_bf16, which
+// subtracts a packed half without unpacking it (seven instructions a pair), shares the matrix
+// pipe: measured, each one held it for about ten cycles.
+__device__ __forceinline__ void split_bf16(const float (&x)[8], bf16x8 (&p)[3]) {
   u32x4 w[3];
 #pragma unroll
   for (int e = 0; e < 4; ++e) {
     float lo = x[2 * e], hi = x[2 * e + 1];
     w[0][e] = pack_bf16(lo, hi);
-    lo = minus_half(w[0][e], c.lo, lo);
-    hi = minus_half(w[0][e], c.hi, hi);
+    lo -= __uint_as_float(w[0][e] << 16);
+    hi -= __uint_as_float(w[0][e] & 0xffff0000u);
     w[1][e] = pack_bf16(lo, hi);
-    w[2][e] = pack_bf16(minus_half(w[1][e], c.lo, lo), minus_half(w[1][e], c.hi, hi));
+    lo -= __uint_as_float(w[1][e] << 16);
+    hi -= __uint_as_float(w[1][e] & 0xffff0000u);
+    w[2][e] = pack_bf16(lo, hi);
   }
 #pragma unroll
   for (int q = 0; q < 3; ++q) p[q] = __builtin_bit_cast(bf16x8, w[q]);
