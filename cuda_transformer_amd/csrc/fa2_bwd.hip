@@ -12,12 +12,13 @@
 //  * dQ stage: a wave owns 32 query rows and keeps q, dO, L and delta of its rows in
 //    registers.  It computes S^T = K Q^T and dP^T = V dO^T (one query row per lane), forms
 //    dS^T in registers and feeds it straight into dQ^T += K^T dS^T.
-//  * dK/dV stage: a wave owns 32 key rows and keeps k and v in registers.  It computes
+//  * dK/dV stage: a wave owns 32 key rows and keeps k and v in registers, as three bfloat16
+//    parts (all its products run on the BF16 matrix pipe, split_bf16.hpp).  It computes
 //    S = Q K^T and dP = dO V^T (one key row per lane) and feeds P and dS straight into
 //    dV^T += dO^T P and dK^T += Q^T dS.  Unlike the reference, causal tiles above the
 //    diagonal are skipped here too (the reference computes kvEnd but never uses it).
-//  * Tiles of the streamed operand (K,V for dQ; Q,dO,L,delta for dK/dV) go
-//    global -> registers -> LDS, double buffered, one barrier per tile.
+//  * dQ streams K and V global -> registers -> LDS, double buffered, one barrier per tile;
+//    dK/dV streams Q, dO, L and delta global -> LDS and splits each stage in LDS.
 //
 // Stored-dS schedule (cta_flash_attention_bwd given a workspace): the reference's dQ stage
 // recomputes S and dP, so the three stages run seven tile GEMMs.  With HBM to spare, the
@@ -27,6 +28,7 @@
 // whole heads (the lower-triangular tiles only when causal); heads are processed in chunks
 // when the caller's workspace cannot hold them all.
 #include "cta_common.hpp"
+#include "split_bf16.hpp"
 
 namespace cta {
 namespace {
@@ -70,24 +72,10 @@ template <> struct BwdTile<32> { static constexpr int BN = 64; static constexpr 
 template <> struct BwdTile<64> { static constexpr int BN = 64; static constexpr int MINW = 2; };
 template <> struct BwdTile<128> { static constexpr int BN = 32; static constexpr int MINW = 1; };
 
-// The dK/dV stage keeps k, v and two accumulator sets per lane, so it streams narrower tiles.
+// Waves per SIMD that the dK/dV stage's registers are held to: k's and v's parts and two
+// accumulator sets are 160 registers at hs 64, 320 at hs 128.
 template <int HS>
-struct DkdvTile;
-template <> struct DkdvTile<32> { static constexpr int BN = 64; static constexpr int MINW = 2; };
-template <> struct DkdvTile<64> { static constexpr int BN = 32; static constexpr int MINW = 2; };
-template <> struct DkdvTile<128> { static constexpr int BN = 32; static constexpr int MINW = 1; };
-
-// Instruction order of a block of MFMAs (sched_group_barrier masks: 0x008 MFMA, 0x100 LDS
-// read): N pairs of MFMAs, each pair followed by one LDS read while I < R.  Preceded by a group
-// of reads, this keeps a fixed number of operand reads in flight ahead of the MFMAs.
-template <int I, int N, int R>
-__device__ __forceinline__ void pin_mfma_pairs() {
-  if constexpr (I < N) {
-    __builtin_amdgcn_sched_group_barrier(0x008, 2, 0);
-    if constexpr (I < R) __builtin_amdgcn_sched_group_barrier(0x100, 1, 0);
-    pin_mfma_pairs<I + 1, N, R>();
-  }
-}
+constexpr int kDkdvMinWaves = HS == 128 ? 1 : 2;
 
 // ------------------------------------------------------------------------------------
 // Stage 2: dQ.  Workgroup = 128 query rows; K/V tiles streamed through LDS.
@@ -305,34 +293,36 @@ constexpr int kDsTileFloats = 1024;
 constexpr int kDsPitch = 40;  // LDS pitch of the per-wave transpose: halves 4 rows apart hit disjoint banks
 
 // ------------------------------------------------------------------------------------
-// Stage 3: dK, dV.  Workgroup = 32 * WAVES key rows (WAVES = 4, or 2 for short causal heads),
-// each wave owning 32 of them and each lane one key row's
-// k and v in registers.  Q, dO, L and delta stream through LDS in stages of BN query rows,
-// copied global -> LDS directly (global_load_lds: no staging registers), double buffered,
-// one barrier per stage.  Query rows past T are read clamped to row T-1 and masked to P = 0.
+// Stage 3: dK, dV.  Workgroup = 128 key rows, each of its four waves owning 32 of them and each
+// lane one key row's k and v, as three bfloat16 parts in registers.  All four products run on
+// the BF16 matrix pipe (split_bf16.hpp; six products of parts, smallest first): 3072 matrix
+// cycles per 32x32 tile at hs 64 where the FP32 MFMA takes 8192, which it kept 85% busy.
 //
-// The Q and dO tiles keep the padded pitch HS + 4, under which both access patterns are
-// free of bank conflicts: the row-segment reads of the S / dP products and the column reads
-// of the dV / dK products.  The async copies fill whole 1 KiB pieces of LDS per wave, so the
-// lanes that land on pad words (or past the dO tile) copy a harmless in-bounds chunk there.
+// Q, dO (O), L and delta stream through LDS in stages of 32 query rows: copied global -> LDS in
+// FP32 (no staging registers) while the stage before is computed, then split once per workgroup
+// into four images in MFMA operand order, Q and dO by rows (S, dP) and by columns (dK, dV).  One
+// image set (48 KiB at hs 64) and one FP32 stage leave room for two workgroups a CU, which hide
+// each other's two barriers a stage; a second image set would leave one.
+// Forward + backward of B4 H32 D64: N4096 causal 7.18 -> 6.24 ms, N8192 55.5 -> 47.3 ms.
 //
 // Heads [bh_base, bh_base + BH) are processed; with STORE_DS every dS tile is also written
-// to dsw (heads indexed from bh_base).  A dS tile goes to a per-wave LDS transpose buffer when
-// it is formed and out to HBM at the start of the next stage, so its stores drain behind a
-// stage of MFMAs rather than in front of the stage's vmcnt wait.
+// to dsw (heads indexed from bh_base), transposed through LDS half a tile at a time.
 //
 // FOLD: delta is not read from a delta stage's output but computed here, per query stage, from
 // the stage's dO tile and an O tile streamed beside it (delta_i = O_i . dO_i, the reference's
 // flash_attention_bwd_delta, flash_attention.cuh:175-213, folded in).  Every key tile of a head
-// recomputes it, and the stage needs a second barrier before delta is read.
+// recomputes it.
 //
 // SPLIT: each work item (key-tile pair, or tile) is run by two workgroups, part 0 and part 1,
 // each over one half of the item's query stages (in the item's stage order, across its passes);
 // every dS tile is still stored once, by the part that forms it.  Part 0 writes its partial dK
 // and dV to dK / dV, part 1 densely to part_ws (dK, then dV, of all BH heads); zeros where a
 // part saw no query stage.  fa2_bwd_dkdv_sum_kernel then adds part 1 to part 0.
-template <int HS, bool CAUSAL, bool STORE_DS, bool FOLD, int WAVES = 4, bool SPLIT = false>
-__global__ __launch_bounds__(64 * WAVES, DkdvTile<HS>::MINW) void fa2_bwd_dkdv_kernel(
+//
+// Sums that the parts cannot vouch for (split_suspect) run the pass again on FP32 MFMAs: a P or
+// dS that is not finite leaves its key's dV or dK not finite, so these two are all that is looked at.
+template <int HS, bool CAUSAL, bool STORE_DS, bool FOLD, bool SPLIT = false>
+__global__ __launch_bounds__(256, kDkdvMinWaves<HS>) void fa2_bwd_dkdv_kernel(
     const float* __restrict__ Q, const float* __restrict__ K, const float* __restrict__ V,
     const float* __restrict__ dO, const float* __restrict__ O, const float* __restrict__ Lg,
     const float* __restrict__ delta, float* __restrict__ dK, float* __restrict__ dV,
@@ -340,23 +330,25 @@ __global__ __launch_bounds__(64 * WAVES, DkdvTile<HS>::MINW) void fa2_bwd_dkdv_k
     RowStrides sk, RowStrides sv, RowStrides sdo, RowStrides so, LStrides sl, RowStrides sdk,
     RowStrides sdv, float scale, float scale_log2, float* __restrict__ part_ws = nullptr,
     int heads_per_xcd = 0) {
-  constexpr int BN = DkdvTile<HS>::BN;
-  constexpr int NSUB = BN / 32;
-  constexpr int THREADS = 64 * WAVES;
+  constexpr int BN = 32, WAVES = 4, THREADS = 64 * WAVES;
   constexpr int BM = 32 * WAVES;  // key rows per workgroup, 32 per wave
-  constexpr int H2 = HS / 2;
-  constexpr int KP = HS + 4;                // LDS pitch of a Q / dO row
-  constexpr int PPT = (BN * KP + 255) / 256;  // 1 KiB async copies per tile
-  constexpr int TILE = PPT * 256;           // a tile's LDS extent: whole copies, rows then pad
-  constexpr int NT = FOLD ? 3 : 2;          // tiles per stage: Q, dO (and O when folding delta)
-  constexpr int PIECES = NT * PPT;
-  constexpr int QG = PIECES * 256;
-  constexpr int RVEC = 64;                  // L and delta of a stage, padded to one wave
-  constexpr int STAGE = QG + 2 * RVEC;
-  constexpr int PER_WAVE = (PIECES + WAVES - 1) / WAVES;
-  static_assert(BN <= RVEC, "one wave copies a stage's L and delta");
-  constexpr int XPOSE = STORE_DS ? WAVES * NSUB * 32 * kDsPitch : 0;
-  __shared__ __attribute__((aligned(16))) float smem[2 * STAGE + XPOSE];
+  constexpr int TILE = BN * HS;     // an FP32 tile: dense rows (convert reads whole runs of them)
+  constexpr int NT = FOLD ? 3 : 2;  // tiles per stage: Q, dO (and O when folding delta)
+  constexpr int RPC = 256 / HS;     // rows of a 1 KiB async copy
+  constexpr int RVEC = 64;  // L and delta of a stage, each padded to one wave
+  // Images, each of three parts: Q by rows, dO by rows, Q by columns, dO by columns, in units of
+  // eight values of one part (16 bytes).  By rows: unit (d8, row) = d 8 d8 .. 8 d8 + 7 of a row,
+  // at d8 * 32 + (row ^ (d8 & 7)).  By columns: unit (d, sh) = the eight query rows that half
+  // sh & 1 takes in step sh >> 1 (16 st + 4 half + 0..3 and + 8..11, the order in which a lane
+  // holds P and dS), at (d/32, sh, d % 32).
+  constexpr int PART = BN * HS * 2, IMAGE = 3 * PART;
+  constexpr int UNITS = BN * HS / 8;  // of one part of one image
+  static_assert(4 * UNITS % THREADS == 0 && UNITS % 64 == 0, "whole waves share an image");
+  constexpr int XPOSE = STORE_DS ? WAVES * 16 * kDsPitch : 0;
+  __shared__ __attribute__((aligned(16))) char images[4 * IMAGE];
+  __shared__ __attribute__((aligned(16))) float raw[NT * TILE];
+  __shared__ __attribute__((aligned(16))) float rvec[2][2 * RVEC];  // by parity of the step
+  __shared__ __attribute__((aligned(16))) float xpose_all[XPOSE > 0 ? XPOSE : 4];
 
   const int tid = threadIdx.x;
   const int lane = tid & 63, wave = wave_index();
@@ -383,31 +375,23 @@ __global__ __launch_bounds__(64 * WAVES, DkdvTile<HS>::MINW) void fa2_bwd_dkdv_k
   const int b = bh / nh, h = bh - b * nh;
 
   const float* Qb = Q + b * sq.b + h * sq.h;
+  const float* Kb = K + b * sk.b + h * sk.h;
+  const float* Vb = V + b * sv.b + h * sv.h;
   const float* dOb = dO + b * sdo.b + h * sdo.h;
   const float* Ob = FOLD ? O + b * so.b + h * so.h : nullptr;
   const float* Lb = Lg + b * sl.b + h * sl.h;
   const float* Db = FOLD ? nullptr : delta + (int64_t)bh * T;
   const int nb = (T + 31) / 32;
-  // Byte offset of each of this lane's copies within its tile's first row of a stage: copy pc
-  // fills floats [256 (pc % PPT), +256) of tile pc / PPT, the lane 4 of them at row f / KP,
-  // column f % KP.  Pad columns and rows past the tile are out of range (no bytes read).
-  int voff[PER_WAVE];
-#pragma unroll
-  for (int u = 0; u < PER_WAVE; ++u) {
-    const int pc = wave + WAVES * u;
-    const int which = pc / PPT;
-    const int f = (pc - which * PPT) * 256 + lane * 4;
-    const int r = f / KP, c = f - r * KP;
-    const int64_t st = which == 0 ? sq.t : (FOLD && which == 2) ? so.t : sdo.t;
-    voff[u] = pc < PIECES && r < BN && c < HS ? (int)((r * st + c) * 4) : (int)0x80000000;
-  }
-  float* xpose = smem + 2 * STAGE + wave * NSUB * 32 * kDsPitch;  // this wave's dS buffers
+  // Byte offset of this lane's 16 bytes in a copy's first row, for the tile's row stride.
+  auto lane_off = [&](int64_t st) { return ((lane * 4 / HS) * (int)st + lane * 4 % HS) * 4; };
+  const int off_q = lane_off(sq.t), off_g = lane_off(sdo.t), off_o = FOLD ? lane_off(so.t) : 0;
+  float* xpose = xpose_all + (STORE_DS ? wave * 16 * kDsPitch : 0);  // this wave's half dS tile
   float* dsh = STORE_DS ? dsw + (int64_t)bh_local * ds_tiles_per_head(T, CAUSAL) * kDsTileFloats
                         : nullptr;
 
-  // Both stage buffers start as zeros, so the rows and pad words no copy writes are finite.
+  // The FP32 stage starts as zeros, so the rows that no copy writes are finite.
 #pragma unroll 4
-  for (int e = 4 * tid; e < 2 * STAGE; e += 4 * THREADS) st4(smem + e, zero4());
+  for (int e = 4 * tid; e < NT * TILE; e += 4 * THREADS) st4(raw + e, zero4());
   __syncthreads();
 
   const int n_pass = kb >= 0 ? 2 : 1;
@@ -423,25 +407,23 @@ __global__ __launch_bounds__(64 * WAVES, DkdvTile<HS>::MINW) void fa2_bwd_dkdv_k
     g0 = part ? (total + 1) / 2 : 0;
     g1 = part ? total : (total + 1) / 2;
   }
+  int slot = 0;  // which of rvec the coming step reads
   for (int pass = 0; pass < n_pass; ++pass) {
   const int kt = kt_of(pass);
   const int j0 = kt * BM + wave * 32;  // first key row of this wave
   const int my_j = j0 + col;
 
-  float kf[H2], vf[H2];
-  if (my_j < T) {
-    const float* kp = K + b * sk.b + h * sk.h + (int64_t)my_j * sk.t + half * H2;
-    const float* vp = V + b * sv.b + h * sv.h + (int64_t)my_j * sv.t + half * H2;
+  // k's and v's parts, the B operands of S and dP: step st, d 16 st + 8 half + 0..7.
+  bf16x8 kp[HS / 16][3], vp[HS / 16][3];
 #pragma unroll
-    for (int c = 0; c < H2 / 4; ++c) {
-      const float4 x = ld4(kp + 4 * c);
-      const float4 y = ld4(vp + 4 * c);
-      kf[4 * c + 0] = x.x; kf[4 * c + 1] = x.y; kf[4 * c + 2] = x.z; kf[4 * c + 3] = x.w;
-      vf[4 * c + 0] = y.x; vf[4 * c + 1] = y.y; vf[4 * c + 2] = y.z; vf[4 * c + 3] = y.w;
-    }
-  } else {
-#pragma unroll
-    for (int c = 0; c < H2; ++c) { kf[c] = 0.0f; vf[c] = 0.0f; }
+  for (int st = 0; st < HS / 16; ++st) {
+    auto load = [&](const float* src, bf16x8 (&p)[3]) {
+      const float4 x = my_j < T ? ld4(src) : zero4(), y = my_j < T ? ld4(src + 4) : zero4();
+      const float v[8] = {x.x, x.y, x.z, x.w, y.x, y.y, y.z, y.w};
+      split_bf16(v, p);
+    };
+    load(Kb + (int64_t)my_j * sk.t + 16 * st + 8 * half, kp[st]);
+    load(Vb + (int64_t)my_j * sv.t + 16 * st + 8 * half, vp[st]);
   }
 
   f32x16 dkacc[HS / 32], dvacc[HS / 32];
@@ -451,43 +433,69 @@ __global__ __launch_bounds__(64 * WAVES, DkdvTile<HS>::MINW) void fa2_bwd_dkdv_k
   const int q_begin = q_begin_of(kt);
   const bool wave_stores = STORE_DS && j0 < T;
 
-  // Async copies of stage `stage` into buffer `buf`.  Piece pc covers floats
-  // [256 pc, 256 pc + 256) of the Q|dO region; wave w copies pieces w, w + WAVES, ...
-  // Each tile of a stage is read through a buffer resource over its valid rows (base and
-  // extent are scalar), so the per-lane offsets above serve every stage; rows past T are out of
-  // range and keep the zeros (or an earlier stage's rows) in LDS, masked to P = 0.
-  auto issue = [&](int stage, int buf) {
-    float* qs = smem + buf * STAGE;
+  // Async copies of a stage into the FP32 tiles.  Each tile is read through a buffer resource
+  // over its valid rows (base and extent are scalar), so the lane's offset serves every copy; rows past T are out of range and leave finite rows in LDS, masked to P = 0.
+  auto issue = [&](int stage, float* rv) {
     const int r0 = stage * BN;
     const int rows = min(BN, T - r0);
-    auto rsrc = [&](const float* base, int64_t st) {
-      return rows_rsrc(base + (int64_t)r0 * st, rows, st, HS);
-    };
-    const __amdgpu_buffer_rsrc_t rq = rsrc(Qb, sq.t), rg = rsrc(dOb, sdo.t);
-    const __amdgpu_buffer_rsrc_t ro = FOLD ? rsrc(Ob, so.t) : rq;
+    auto copy = [&](const float* base, int64_t st, int off, float* tile) {
+      const __amdgpu_buffer_rsrc_t rs = rows_rsrc(base + (int64_t)r0 * st, rows, st, HS);
 #pragma unroll
-    for (int u = 0; u < PER_WAVE; ++u) {
-      const int pc = wave + WAVES * u;
-      if (pc < PIECES) {
-        const int which = pc / PPT;  // 0: Q, 1: dO, 2: O (FOLD)
-        async_copy16_buffer(which == 0 ? rq : which == 1 ? rg : ro, voff[u], qs + pc * 256);
+      for (int u = 0; u < BN / RPC / WAVES; ++u) {
+        const int pc = wave + WAVES * u;
+        async_copy16_buffer(rs, off + pc * RPC * (int)st * 4, tile + pc * 256);
       }
-    }
+    };
+    copy(Qb, sq.t, off_q, raw);
+    copy(dOb, sdo.t, off_g, raw + TILE);
+    if (FOLD) copy(Ob, so.t, off_o, raw + 2 * TILE);
     if (wave == 0) {  // lanes past BN fill the padding
       const int64_t i = min(r0 + lane, T - 1);
-      async_copy4(Lb + i * sl.t, qs + QG);
-      if (!FOLD) async_copy4(Db + i, qs + QG + RVEC);
+      async_copy4(Lb + i * sl.t, rv);
+      if (!FOLD) async_copy4(Db + i, rv + RVEC);
     }
   };
-  // FOLD: delta of the stage in buffer `st` from its O and dO tiles, THREADS / BN lanes per row,
-  // into the stage's delta slot.  Rows past T hold row T - 1 (their P is masked to 0).
-  auto fold_delta = [&](float* st) {
+  // The four images from the FP32 tiles, one unit (three parts) at a time.
+  auto convert = [&]() {
+#pragma unroll
+    for (int u = 0; u < 4 * UNITS / THREADS; ++u) {
+      // unit f of image img: a constant where a step of the workgroup stays in one image
+      const int img = UNITS >= THREADS
+                          ? THREADS * u / UNITS
+                          : THREADS / UNITS * u + __builtin_amdgcn_readfirstlane(tid / UNITS);
+      const int f = UNITS >= THREADS ? tid + THREADS * u % UNITS : tid % UNITS;
+      const float* src = raw + (img & 1) * TILE;
+      float x[8];
+      int at;
+      if (img < 2) {
+        const int r = f / (HS / 8), d8 = f % (HS / 8);
+        const float4 lo = ld4(src + r * HS + 8 * d8), hi = ld4(src + r * HS + 8 * d8 + 4);
+        x[0] = lo.x; x[1] = lo.y; x[2] = lo.z; x[3] = lo.w;
+        x[4] = hi.x; x[5] = hi.y; x[6] = hi.z; x[7] = hi.w;
+        at = d8 * 32 + (r ^ (d8 & 7));
+      } else {
+        const int d = f % HS, sh = f / HS;
+        const float* c = src + (16 * (sh >> 1) + 4 * (sh & 1)) * HS + d;
+#pragma unroll
+        for (int j = 0; j < 8; ++j) x[j] = c[(8 * (j >> 2) + (j & 3)) * HS];
+        at = (d >> 5) * 128 + sh * 32 + (d & 31);
+      }
+      bf16x8 p[3];
+      split_bf16(x, p);
+#pragma unroll
+      for (int q = 0; q < 3; ++q)
+        *reinterpret_cast<bf16x8*>(images + img * IMAGE + q * PART + at * 16) = p[q];
+    }
+  };
+  // FOLD: delta of the stage from its O and dO tiles, THREADS / BN lanes per row.  Rows past T
+  // are masked (P = 0).
+  auto fold_delta = [&](float* rv) {
     constexpr int LPR = THREADS / BN;  // lanes per row (consecutive lanes of one wave)
     constexpr int DPL = HS / LPR;      // d values per lane
     static_assert(THREADS % BN == 0 && DPL % 4 == 0 && LPR <= 64, "delta split");
     const int r = tid / LPR, seg = tid % LPR;
-    const float* orow = st + 2 * TILE + r * KP + seg * DPL;
-    const float* grow = st + TILE + r * KP + seg * DPL;
+    const float* orow = raw + 2 * TILE + r * HS + seg * DPL;
+    const float* grow = raw + TILE + r * HS + seg * DPL;
     float acc = 0.0f;
 #pragma unroll
     for (int c = 0; c < DPL / 4; ++c) {
@@ -499,24 +507,63 @@ __global__ __launch_bounds__(64 * WAVES, DkdvTile<HS>::MINW) void fa2_bwd_dkdv_k
     }
 #pragma unroll
     for (int off = LPR / 2; off >= 1; off >>= 1) acc += __shfl_xor(acc, off);
-    if (seg == 0) st[QG + RVEC + r] = acc;
+    if (seg == 0) rv[RVEC + r] = acc;
   };
   // Tiles whose every query row precedes every key row are skipped (dS = 0, nothing stored).
   auto live = [&](int ii0) { return ii0 < T && !(CAUSAL && ii0 + 31 < j0); };
-  // Copy the dS tiles of `stage` from the transpose buffers to the workspace.
-  auto flush = [&](int stage) {
+  // S (query rows ii0 + R(r, half), key my_j) -> P = e^{S - L}; masked entries and key rows past
+  // T give exactly 0.
+  auto probabilities = [&](f32x16& sacc, int ii0, const float* ls) {
+    // A separate block behind a wave-uniform branch: inside the exponential loop the test is
+    // if-converted into per-element predication that every tile pays for.
+    if ((CAUSAL && ii0 < j0 + 31) || (ii0 + 32 > T) || (j0 + 32 > T)) {
+      asm volatile("");  // a side effect keeps the block from being speculated into selects
 #pragma unroll
-    for (int sub = 0; sub < NSUB; ++sub) {
-      const int ii0 = stage * BN + sub * 32;
-      if (!live(ii0)) continue;
-      const float* xw = xpose + sub * 32 * kDsPitch;
-      float* gt = dsh + ds_tile_index(ii0 / 32, j0 / 32, nb, CAUSAL) * kDsTileFloats;
-      wave_lds_fence();
-#pragma unroll
-      for (int g = 0; g < 4; ++g)
-        st4_stream(gt + 256 * g + 4 * lane, ld4(xw + col * kDsPitch + 8 * g + 4 * half));
-      wave_lds_fence();
+      for (int r = 0; r < 16; ++r) {
+        const int i = ii0 + mfma_row(r, half);
+        if ((CAUSAL && my_j > i) || i >= T || my_j >= T) sacc[r] = -INFINITY;
+      }
     }
+#pragma unroll
+    for (int g = 0; g < 4; ++g) {
+      const float4 lv = ld4(ls + 8 * g + 4 * half);
+      const float lr[4] = {lv.x, lv.y, lv.z, lv.w};
+#pragma unroll
+      for (int e = 0; e < 4; ++e)
+        sacc[4 * g + e] = fast_exp2(fmaf(sacc[4 * g + e], scale_log2, -lr[e] * kLog2e));
+    }
+  };
+  // dP -> dS = P (dP - delta).  Rounded to FP32 before it is split: fused into the split's first
+  // subtraction (where nothing stores dS) it would give the schedules different bits.
+  auto score_gradients = [&](const f32x16& p, f32x16& pacc, const float* ds) {
+#pragma clang fp contract(off)
+#pragma unroll
+    for (int g = 0; g < 4; ++g) {
+      const float4 dv = ld4(ds + 8 * g + 4 * half);
+      const float dr[4] = {dv.x, dv.y, dv.z, dv.w};
+#pragma unroll
+      for (int e = 0; e < 4; ++e) pacc[4 * g + e] = p[4 * g + e] * (pacc[4 * g + e] - dr[e]);
+    }
+  };
+  // Lane (col, half) holds dS[ii0 + R(r, half)][j0 + col]: through the wave's transpose buffer
+  // as [query][key], 16 queries at a time, and out one query row per lane in whole 256-byte runs.
+  auto store_ds = [&](const f32x16& dsv, int ii0) {
+    float* gt = dsh + ds_tile_index(ii0 / 32, j0 / 32, nb, CAUSAL) * kDsTileFloats;
+    const int gs = lane >> 5, hs = (lane >> 4) & 1, c = lane & 15;
+#pragma unroll
+    for (int hh = 0; hh < 2; ++hh) {
+      wave_lds_fence();
+#pragma unroll
+      for (int r = 0; r < 8; ++r) xpose[mfma_row(r, half) * kDsPitch + col] = dsv[8 * hh + r];
+      wave_lds_fence();
+#pragma unroll
+      for (int k = 0; k < 2; ++k) {
+        const int g = 2 * k + gs;
+        st4_stream(gt + 256 * g + 4 * (32 * hs + 16 * hh + c),
+                   ld4(xpose + c * kDsPitch + 8 * g + 4 * hs));
+      }
+    }
+    wave_lds_fence();
   };
 
   // Stage order.  With a causal mask the first (long) pass walks its query stages downward
@@ -532,151 +579,155 @@ __global__ __launch_bounds__(64 * WAVES, DkdvTile<HS>::MINW) void fa2_bwd_dkdv_k
   // (the long tile of a pair walks down: a property of the tile, so single tiles match pairs)
   const bool down = CAUSAL && kt <= n_ktiles - 1 - kt;
   auto stage_at = [&](int i) { return down ? n_stages - 1 - i : q_begin + i; };
-  if (i_begin < i_end) issue(stage_at(i_begin), 0);
-  vm_wait_all();
-  __syncthreads();
+  if (i_begin < i_end) issue(stage_at(i_begin), rvec[slot]);
 
   for (int i = i_begin; i < i_end; ++i) {
-    const int s = stage_at(i);
-    const int buf = (i - i_begin) & 1;
-    if (i + 1 < i_end) issue(stage_at(i + 1), buf ^ 1);
-    if (wave_stores && i > i_begin) flush(stage_at(i - 1));
-    if (FOLD) {
-      fold_delta(smem + buf * STAGE);
-      __syncthreads();
-    }
-    const float* qs = smem + buf * STAGE;
-    const float* gs = qs + TILE;
-    const float* ls = qs + QG;
-    const float* ds = ls + RVEC;
-
-#pragma unroll
-    for (int sub = 0; sub < NSUB; ++sub) {
-      const int ii0 = s * BN + sub * 32;
-      if (!live(ii0)) continue;
-
-      // S and dP tiles: lane holds column my_j, rows ii0 + R(r, half)
-      f32x16 sacc = zero16(), pacc = zero16();
-      const float* qrow = qs + (sub * 32 + col) * KP + half * H2;
-      const float* grow = gs + (sub * 32 + col) * KP + half * H2;
-#pragma unroll
-      for (int c = 0; c < H2 / 4; ++c) {
-        const float4 qv = ld4(qrow + 4 * c);
-        const float4 gv = ld4(grow + 4 * c);
-        sacc = mfma32(qv.x, kf[4 * c + 0], sacc);
-        pacc = mfma32(gv.x, vf[4 * c + 0], pacc);
-        sacc = mfma32(qv.y, kf[4 * c + 1], sacc);
-        pacc = mfma32(gv.y, vf[4 * c + 1], pacc);
-        sacc = mfma32(qv.z, kf[4 * c + 2], sacc);
-        pacc = mfma32(gv.z, vf[4 * c + 2], pacc);
-        sacc = mfma32(qv.w, kf[4 * c + 3], sacc);
-        pacc = mfma32(gv.w, vf[4 * c + 3], pacc);
-      }
-
-      // Masked entries (and, when storing dS, key rows past T, so a stored tile is exactly 0
-      // there) become -inf, so P = 2^-inf = 0 below.  A separate block behind a wave-uniform
-      // branch: inside the exponential loop the test is if-converted into per-element
-      // predication that every tile pays for.
-      if ((CAUSAL && ii0 < j0 + 31) || (ii0 + 32 > T) || (STORE_DS && j0 + 32 > T)) {
-        asm volatile("");  // a side effect keeps the block from being speculated into selects
-#pragma unroll
-        for (int r = 0; r < 16; ++r) {
-          const int i = ii0 + mfma_row(r, half);
-          if ((CAUSAL && my_j > i) || i >= T || (STORE_DS && my_j >= T)) sacc[r] = -INFINITY;
-        }
-      }
-      // P = e^{S - L}; masked entries are exactly 0.
-#pragma unroll
-      for (int g = 0; g < 4; ++g) {
-        const float4 lv = ld4(ls + sub * 32 + 8 * g + 4 * half);
-        const float lr[4] = {lv.x, lv.y, lv.z, lv.w};
-#pragma unroll
-        for (int e = 0; e < 4; ++e) {
-          const int r = 4 * g + e;
-          sacc[r] = fast_exp2(fmaf(sacc[r], scale_log2, -lr[e] * kLog2e));
-        }
-      }
-
-      // dV^T += dO^T P is issued before dS is formed, so the dS arithmetic and its transpose
-      // writes overlap these MFMAs; then dK^T += Q^T dS.  One product at a time keeps at most
-      // one set of LDS operands in flight.
-      //
-      // The A operand of step kk is (query row R(kk, half), column d*32 + col) of the dO or Q
-      // tile.  For HS <= 64 it is addressed from one lane base pointer plus a compile-time row
-      // offset (8 (kk/4) + kk%4), which the LDS reads carry as immediates: per-read row
-      // arithmetic held registers at the 256-VGPR limit and forced each read to wait just
-      // before its MFMA.  With the registers free, the reads are pinned several MFMA pairs
-      // ahead.  HS = 128 (one wave per SIMD) measured faster with the per-read form.
-      const float* gcol = gs + (sub * 32 + 4 * half) * KP + col;
-      const float* qcol = qs + (sub * 32 + 4 * half) * KP + col;
-      auto a_op = [&](const float* tile, const float* lane_col, int kk, int d) {
-        return HS == 128 ? tile[(sub * 32 + mfma_row(kk, half)) * KP + d * 32 + col]
-                         : lane_col[(8 * (kk >> 2) + (kk & 3)) * KP + d * 32];
-      };
-#pragma unroll
-      for (int kk = 0; kk < 16; ++kk) {
-#pragma unroll
-        for (int d = 0; d < HS / 32; ++d) dvacc[d] = mfma32(a_op(gs, gcol, kk, d), sacc[kk], dvacc[d]);
-      }
-#pragma unroll
-      for (int g = 0; g < 4; ++g) {
-        const float4 dv = ld4(ds + sub * 32 + 8 * g + 4 * half);
-        const float dr[4] = {dv.x, dv.y, dv.z, dv.w};
-#pragma unroll
-        for (int e = 0; e < 4; ++e) pacc[4 * g + e] = sacc[4 * g + e] * (pacc[4 * g + e] - dr[e]);
-      }
-      // L's four reads and four dO pairs ahead of the first MFMA pair, then one read (dO
-      // operands, then delta) after each pair.
-      if (HS == 64) {
-        __builtin_amdgcn_sched_group_barrier(0x100, 4 + 4, 0);
-        pin_mfma_pairs<0, 16, 16>();
-      }
-
-      // Lane (col, half) holds dS[ii0 + R(r, half)][j0 + col]: into the transpose buffer as
-      // [query][key]; flush() reads it back one query row per lane.  A wave's LDS operations
-      // complete in order, so no barrier separates the write, the read and the next write.
-      if (wave_stores) {
-        float* xw = xpose + sub * 32 * kDsPitch;
-#pragma unroll
-        for (int r = 0; r < 16; ++r) xw[mfma_row(r, half) * kDsPitch + col] = pacc[r];
-      }
-
-#pragma unroll
-      for (int kk = 0; kk < 16; ++kk) {
-#pragma unroll
-        for (int d = 0; d < HS / 32; ++d) dkacc[d] = mfma32(a_op(qs, qcol, kk, d), pacc[kk], dkacc[d]);
-      }
-      if (HS == 64) {  // four Q pairs ahead
-        __builtin_amdgcn_sched_group_barrier(0x100, 4, 0);
-        pin_mfma_pairs<0, 16, 12>();
-      }
-    }
-
+    // the stage's copies have landed, and every wave is done with the images
     vm_wait_all();
     __syncthreads();
+    convert();
+    float* const rv = rvec[slot];
+    if (FOLD) fold_delta(rv);
+    slot ^= 1;
+    __syncthreads();
+    if (i + 1 < i_end) issue(stage_at(i + 1), rvec[slot]);
+
+    const int ii0 = stage_at(i) * BN;
+    if (!live(ii0)) continue;
+
+    // S and dP tiles: lane holds column my_j, rows ii0 + R(r, half)
+    f32x16 sacc = zero16(), pacc = zero16();
+#pragma unroll
+    for (int st = 0; st < HS / 16; ++st) {
+      const int d8 = 2 * st + half;
+      const char* at = images + (d8 * 32 + (col ^ (d8 & 7))) * 16;
+      bf16x8 qa[3], ga[3];
+#pragma unroll
+      for (int q = 2; q >= 0; --q) {
+        qa[q] = *reinterpret_cast<const bf16x8*>(at + q * PART);
+        ga[q] = *reinterpret_cast<const bf16x8*>(at + IMAGE + q * PART);
+      }
+#pragma unroll
+      for (int p = 0; p < 6; ++p) {
+        sacc = mfma_bf16(qa[kSplitA[p]], kp[st][kSplitB[p]], sacc);
+        pacc = mfma_bf16(ga[kSplitA[p]], vp[st][kSplitB[p]], pacc);
+      }
+    }
+    // X^T += (image's columns) Y over the 32 query rows, two steps of 16
+    auto accumulate = [&](f32x16 (&acc)[HS / 32], const char* image, const f32x16& y) {
+#pragma unroll
+      for (int st = 0; st < 2; ++st) {
+        float x[8];
+#pragma unroll
+        for (int e = 0; e < 8; ++e) x[e] = y[8 * st + e];
+        bf16x8 yp[3];
+        split_bf16(x, yp);
+#pragma unroll
+        for (int d0 = 0; d0 < HS / 32; d0 += 2) {
+          constexpr int ND = HS / 32 < 2 ? 1 : 2;  // two chains
+          bf16x8 a[ND][3];
+#pragma unroll
+          for (int d = 0; d < ND; ++d)
+#pragma unroll
+            for (int q = 2; q >= 0; --q)
+              a[d][q] = *reinterpret_cast<const bf16x8*>(
+                  image + q * PART + ((d0 + d) * 128 + (2 * st + half) * 32 + col) * 16);
+#pragma unroll
+          for (int p = 0; p < 6; ++p)
+#pragma unroll
+            for (int d = 0; d < ND; ++d)
+              acc[d0 + d] = mfma_bf16(a[d][kSplitA[p]], yp[kSplitB[p]], acc[d0 + d]);
+        }
+      }
+    };
+    probabilities(sacc, ii0, rv);
+    accumulate(dvacc, images + 3 * IMAGE, sacc);
+    score_gradients(sacc, pacc, rv + RVEC);
+    if (wave_stores) store_ds(pacc, ii0);
+    accumulate(dkacc, images + 2 * IMAGE, pacc);
   }
-  if (wave_stores && i_end > i_begin) flush(stage_at(i_end - 1));
+
+  bool odd = false;
+#pragma unroll
+  for (int d = 0; d < HS / 32; ++d) odd |= split_suspect(dkacc[d]) || split_suspect(dvacc[d]);
+  vm_wait_all();  // dS tiles that a second run stores again are stored in order
+  if (__syncthreads_or(odd)) {
+#pragma unroll
+    for (int d = 0; d < HS / 32; ++d) { dkacc[d] = zero16(); dvacc[d] = zero16(); }
+    for (int i = i_begin; i < i_end; ++i) {
+      const int ii0 = stage_at(i) * BN;
+      float* const rv = rvec[slot];
+      __syncthreads();
+      for (int f = tid; f < BN * HS / 4; f += THREADS) {
+        const int r = f / (HS / 4), c4 = f % (HS / 4) * 4;
+        const int64_t t = ii0 + r;
+        st4(raw + r * HS + c4, t < T ? ld4(Qb + t * sq.t + c4) : zero4());
+        st4(raw + TILE + r * HS + c4, t < T ? ld4(dOb + t * sdo.t + c4) : zero4());
+        if (FOLD) st4(raw + 2 * TILE + r * HS + c4, t < T ? ld4(Ob + t * so.t + c4) : zero4());
+      }
+      if (tid < BN) {
+        const int64_t t = min(ii0 + tid, T - 1);
+        rv[tid] = Lb[t * sl.t];
+        if (!FOLD) rv[RVEC + tid] = Db[t];
+      }
+      __syncthreads();
+      if (FOLD) {
+        fold_delta(rv);
+        __syncthreads();
+      }
+      if (!live(ii0)) continue;
+      f32x16 sacc = zero16(), pacc = zero16();
+      const int64_t jc = min(my_j, T - 1);
+      const float* k = Kb + jc * sk.t + half * (HS / 2);
+      const float* v = Vb + jc * sv.t + half * (HS / 2);
+      const float* qrow = raw + col * HS + half * (HS / 2);
+#pragma unroll 2
+      for (int c = 0; c < HS / 2; c += 4) {
+        const float4 q4 = ld4(qrow + c), g4 = ld4(qrow + TILE + c), k4 = ld4(k + c), v4 = ld4(v + c);
+        sacc = mfma32(q4.x, k4.x, sacc);
+        pacc = mfma32(g4.x, v4.x, pacc);
+        sacc = mfma32(q4.y, k4.y, sacc);
+        pacc = mfma32(g4.y, v4.y, pacc);
+        sacc = mfma32(q4.z, k4.z, sacc);
+        pacc = mfma32(g4.z, v4.z, pacc);
+        sacc = mfma32(q4.w, k4.w, sacc);
+        pacc = mfma32(g4.w, v4.w, pacc);
+      }
+      probabilities(sacc, ii0, rv);
+      score_gradients(sacc, pacc, rv + RVEC);
+      if (wave_stores) store_ds(pacc, ii0);
+#pragma unroll
+      for (int d = 0; d < HS / 32; ++d)
+#pragma unroll
+        for (int kk = 0; kk < 16; ++kk) {
+          const float* a = raw + mfma_row(kk, half) * HS + d * 32 + col;
+          dvacc[d] = mfma32(a[TILE], sacc[kk], dvacc[d]);
+          dkacc[d] = mfma32(a[0], pacc[kk], dkacc[d]);
+        }
+    }
+    __syncthreads();
+  }
 
   if (my_j < T) {
-    float* kp = dK + b * sdk.b + h * sdk.h + (int64_t)my_j * sdk.t;
-    float* vp = dV + b * sdv.b + h * sdv.h + (int64_t)my_j * sdv.t;
+    float* dkp = dK + b * sdk.b + h * sdk.h + (int64_t)my_j * sdk.t;
+    float* dvp = dV + b * sdv.b + h * sdv.h + (int64_t)my_j * sdv.t;
     if (SPLIT && part) {
-      kp = part_ws + ((int64_t)bh * T + my_j) * HS;
-      vp = kp + (int64_t)(bh_base + BH) * T * HS;
+      dkp = part_ws + ((int64_t)bh * T + my_j) * HS;
+      dvp = dkp + (int64_t)(bh_base + BH) * T * HS;
     }
 #pragma unroll
     for (int d = 0; d < HS / 32; ++d) {
 #pragma unroll
       for (int g = 0; g < 4; ++g) {
         const int dc = d * 32 + 8 * g + 4 * half;
-        st4(kp + dc, make_float4(dkacc[d][4 * g + 0] * scale, dkacc[d][4 * g + 1] * scale,
-                                 dkacc[d][4 * g + 2] * scale, dkacc[d][4 * g + 3] * scale));
-        st4(vp + dc, make_float4(dvacc[d][4 * g + 0], dvacc[d][4 * g + 1], dvacc[d][4 * g + 2],
-                                 dvacc[d][4 * g + 3]));
+        st4(dkp + dc, make_float4(dkacc[d][4 * g + 0] * scale, dkacc[d][4 * g + 1] * scale,
+                                  dkacc[d][4 * g + 2] * scale, dkacc[d][4 * g + 3] * scale));
+        st4(dvp + dc, make_float4(dvacc[d][4 * g + 0], dvacc[d][4 * g + 1], dvacc[d][4 * g + 2],
+                                  dvacc[d][4 * g + 3]));
       }
     }
   }
-  }  // pass: the stage loop ended on a barrier, so the next pass may refill LDS
+  }  // pass: the check above is a barrier, so the next pass may refill LDS
 }
 
 // dK += part 1's dK, dV += part 1's dV, row by row in a fixed order (part 0, then part 1), after
@@ -948,7 +999,7 @@ void launch_dq(const float* q, const float* k, const float* v, const float* d_o,
 
 // dK/dV for heads [bh_base, bh_base + n_heads), written through strides sdk / sdv; with
 // STORE_DS the dS tiles go to dsw; with FOLD delta comes from O (strides so) instead of the
-// delta array.  Four waves (128 keys) per workgroup, or two for short causal heads.
+// delta array.  Four waves (128 keys) per workgroup.
 // part_ws (heads [0, n_heads) with bh_base = 0 only): run the split form and its sum pass.
 template <int HS, bool CAUSAL, bool STORE_DS, bool FOLD = false>
 void launch_dkdv(const float* q, const float* k, const float* v, const float* d_o,
@@ -957,40 +1008,26 @@ void launch_dkdv(const float* q, const float* k, const float* v, const float* d_
                  RowStrides sdo, LStrides sl, RowStrides sdk, RowStrides sdv, float scale,
                  hipStream_t st, const float* o = nullptr, RowStrides so = {},
                  float* part_ws = nullptr) {
-  auto run = [&]<int WAVES>() {
-    const int n_ktiles = (T + 32 * WAVES - 1) / (32 * WAVES);
-    const int64_t items = (int64_t)(CAUSAL ? (n_ktiles + 1) / 2 : n_ktiles) * n_heads;
-    if (part_ws != nullptr) {
-      hipLaunchKernelGGL((fa2_bwd_dkdv_kernel<HS, CAUSAL, STORE_DS, FOLD, WAVES, true>),
-                         dim3(xcd_grid(2 * items)), dim3(64 * WAVES), 0, st, q, k, v, d_o, o, l,
-                         delta, dk, dv, dsw, nh, T, bh_base, n_heads, n_ktiles, sq, sk, sv, sdo,
-                         so, sl, sdk, sdv, scale, scale * kLog2e, part_ws);
-      const int64_t rows = (int64_t)n_heads * T;
-      hipLaunchKernelGGL((fa2_bwd_dkdv_sum_kernel<HS>),
-                         dim3((unsigned)((rows * (HS / 4) + 255) / 256)), dim3(256), 0, st, dk,
-                         dv, part_ws, nh, T, rows, sdk, sdv);
-      return;
-    }
-    const int lpt = CAUSAL ? lpt_heads(n_heads, n_ktiles, WAVES, DkdvTile<HS>::MINW) : 0;
-    hipLaunchKernelGGL((fa2_bwd_dkdv_kernel<HS, CAUSAL, STORE_DS, FOLD, WAVES>),
-                       dim3(lpt > 0 ? (unsigned)(n_heads * n_ktiles) : xcd_grid(items)),
-                       dim3(64 * WAVES), 0, st, q, k, v, d_o, o, l, delta, dk, dv, dsw, nh, T,
-                       bh_base, n_heads, n_ktiles, sq, sk, sv, sdo, so, sl, sdk, sdv, scale,
-                       scale * kLog2e, nullptr, lpt);
-  };
-  // Short causal heads (hs 64, T <= 1024) run two waves (64 keys) per workgroup: the half-empty
-  // diagonal blocks idle fewer waves at each stage's barrier and the pairs balance over more,
-  // smaller workgroups.  A/B in one process: +17% at T = 256 (the GPT step's shape), +11% at
-  // 512, +4% at 1024, equal at 2048; 26% slower non-causal at 256 and 39% at config 2, where
-  // each key now costs twice the Q / dO staging.  Every schedule (stored dS, recompute, delta
-  // folded) takes the same shape, so their dK / dV stay bitwise equal.
-  if constexpr (HS == 64 && CAUSAL) {
-    if (T <= 1024) {
-      run.template operator()<2>();
-      return;
-    }
+  constexpr int WAVES = 4;
+  const int n_ktiles = (T + 32 * WAVES - 1) / (32 * WAVES);
+  const int64_t items = (int64_t)(CAUSAL ? (n_ktiles + 1) / 2 : n_ktiles) * n_heads;
+  if (part_ws != nullptr) {
+    hipLaunchKernelGGL((fa2_bwd_dkdv_kernel<HS, CAUSAL, STORE_DS, FOLD, true>),
+                       dim3(xcd_grid(2 * items)), dim3(64 * WAVES), 0, st, q, k, v, d_o, o, l,
+                       delta, dk, dv, dsw, nh, T, bh_base, n_heads, n_ktiles, sq, sk, sv, sdo,
+                       so, sl, sdk, sdv, scale, scale * kLog2e, part_ws);
+    const int64_t rows = (int64_t)n_heads * T;
+    hipLaunchKernelGGL((fa2_bwd_dkdv_sum_kernel<HS>),
+                       dim3((unsigned)((rows * (HS / 4) + 255) / 256)), dim3(256), 0, st, dk,
+                       dv, part_ws, nh, T, rows, sdk, sdv);
+    return;
   }
-  run.template operator()<4>();
+  const int lpt = CAUSAL ? lpt_heads(n_heads, n_ktiles, WAVES, kDkdvMinWaves<HS>) : 0;
+  hipLaunchKernelGGL((fa2_bwd_dkdv_kernel<HS, CAUSAL, STORE_DS, FOLD>),
+                     dim3(lpt > 0 ? (unsigned)(n_heads * n_ktiles) : xcd_grid(items)),
+                     dim3(64 * WAVES), 0, st, q, k, v, d_o, o, l, delta, dk, dv, dsw, nh, T,
+                     bh_base, n_heads, n_ktiles, sq, sk, sv, sdo, so, sl, sdk, sdv, scale,
+                     scale * kLog2e, nullptr, lpt);
 }
 
 // part_ws (heads [0, n_heads) with bh_base = 0 only): run the split form and its sum pass.
@@ -1031,16 +1068,16 @@ void launch_dq_ds(const float* k, const float* dsw, float* dq, int nh, int T, in
 
 // The stored-dS dK/dV stage splits each item's query stages over two workgroups when its grid
 // would hold fewer than two waves per SIMD (1024 SIMDs) and a full column of queries gives each
-// part at least kSplitMinStages stages (T >= 1024 at 32-row stages), as the forward does.
+// part at least kSplitMinStages stages (T >= 1024; 2048 at hs 32, whose stages are half the work),
+// as the forward does.
 constexpr int kSimds = 1024;
 constexpr int kSplitMinStages = 16;
 
 template <int HS, bool CAUSAL>
 bool dkdv_split(int T, int BH) {
-  const int waves = (HS == 64 && CAUSAL && T <= 1024) ? 2 : 4;
-  const int n_ktiles = (T + 32 * waves - 1) / (32 * waves);
+  const int n_ktiles = (T + 127) / 128;
   const int64_t items = (int64_t)(CAUSAL ? (n_ktiles + 1) / 2 : n_ktiles) * BH;
-  return items * waves < 2 * kSimds && T / DkdvTile<HS>::BN >= 2 * kSplitMinStages;
+  return items * 4 < 2 * kSimds && T / (HS == 32 ? 64 : 32) >= 2 * kSplitMinStages;
 }
 
 // Runs f.template operator()<HS, CAUSAL>() for the runtime head size and mask flag.

@@ -49,3 +49,46 @@ def test_forward_outside_the_split_range(cuda, T, causal, D):
     q, k, v = _qkv(1, 2, T, D, T + D)
     o, _ = flash_attention_fwd(q.to(cuda), k.to(cuda), (v * 2.0 ** -120).to(cuda), causal)
     assert _rel(o.cpu().double() * 2.0 ** 120, ref) <= 1e-6
+
+
+def _grads(cuda, q, k, v, dy, causal):
+    from cuda_autograd_fns import CudaFlashAttention
+
+    leaves = [x.to(cuda).requires_grad_() for x in (q, k, v)]
+    o, _ = CudaFlashAttention.apply(*leaves, causal)
+    return torch.autograd.grad(o, leaves, dy.to(cuda))
+
+
+@pytest.mark.parametrize("D", [32, 64, 128])
+@pytest.mark.parametrize("T,causal", [(1, True), (33, False), (130, True), (160, False), (1100, True)])
+def test_gradients_against_float64(cuda, T, causal, D):
+    """FP32 sums of a few thousand terms: a few units of 2^-24 in the 2-norm (T = 1: dQ and dK are
+    rounding noise about zero, so only dV is compared)."""
+    q, k, v, dy = _qkv(1, 2, T, D, T + D, 4)
+    _, *ref = _ref(q, k, v, causal, dy)
+    for name, x, r in zip("qkv", _grads(cuda, q, k, v, dy, causal), ref):
+        if T > 1 or name == "v":
+            assert _rel(x, r) <= 1.5e-6, (name, _rel(x, r))
+
+
+@pytest.mark.parametrize("D", [32, 64, 128])
+@pytest.mark.parametrize("T,causal", [(33, True), (160, False), (300, True)])
+def test_gradients_outside_the_split_range(cuda, T, causal, D):
+    q, k, v, dy = _qkv(1, 2, T, D, T + D, 4)
+    _, *ref = _ref(q, k, v, causal, dy)
+    # gradients of 2^-110: as accurate as ordinary ones
+    for x, r in zip(_grads(cuda, q, k, v, dy * 2.0 ** -110, causal), ref):
+        assert _rel(x.cpu().double() * 2.0 ** 110, r) <= 1.5e-6
+    # an infinite entry of dO: the keys its row sees get an infinite (not NaN) dV there; the
+    # other head, and every other column of dV, are untouched
+    i, d = T // 2, 3
+    dy[0, 0, i, d] = float("inf")
+    dq, dk, dv = (x.cpu() for x in _grads(cuda, q, k, v, dy, causal))
+    sees = torch.arange(T) <= (i if causal else T)
+    assert torch.all(dv[0, 0, sees, d] == float("inf"))
+    dv[0, 0, :, d] = ref[2][0, 0, :, d].float()  # a masked key of the same tile: 0 x inf
+    assert _rel(dv, ref[2]) <= 1.5e-6
+    for x, r in ((dq, ref[0]), (dk, ref[1])):
+        assert _rel(x[0, 1], r[0, 1]) <= 1.5e-6
+    rows = torch.arange(T) != i
+    assert _rel(dq[0, 0, rows], ref[0][0, 0, rows]) <= 1.5e-6
