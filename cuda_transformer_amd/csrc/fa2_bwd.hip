@@ -303,7 +303,9 @@ constexpr int kDsPitch = 40;  // LDS pitch of the per-wave transpose: halves 4 r
 // into four images in MFMA operand order, Q and dO by rows (S, dP) and by columns (dK, dV).  One
 // image set (48 KiB at hs 64) and one FP32 stage leave room for two workgroups a CU, which hide
 // each other's two barriers a stage; a second image set would leave one.
-// Forward + backward of B4 H32 D64: N4096 causal 7.18 -> 6.24 ms, N8192 55.5 -> 47.3 ms.
+// B4 H32 N4096 D64 causal: 4.2 -> 3.2 ms, 45% of the matrix cycles; B2 H16 T1999 D128 0.52 ms.
+// The rest is VALU work (the splits and the softmax, about 600 instructions a tile, in long runs
+// between the MFMAs), the barriers and the chip's power limit.
 //
 // Heads [bh_base, bh_base + BH) are processed; with STORE_DS every dS tile is also written
 // to dsw (heads indexed from bh_base), transposed through LDS half a tile at a time.
@@ -431,7 +433,6 @@ __global__ __launch_bounds__(256, kDkdvMinWaves<HS>) void fa2_bwd_dkdv_kernel(
   for (int d = 0; d < HS / 32; ++d) { dkacc[d] = zero16(); dvacc[d] = zero16(); }
 
   const int q_begin = q_begin_of(kt);
-  const bool wave_stores = STORE_DS && j0 < T;
 
   // Async copies of a stage into the FP32 tiles.  Each tile is read through a buffer resource
   // over its valid rows (base and extent are scalar), so the lane's offset serves every copy; rows past T are out of range and leave finite rows in LDS, masked to P = 0.
@@ -509,8 +510,9 @@ __global__ __launch_bounds__(256, kDkdvMinWaves<HS>) void fa2_bwd_dkdv_kernel(
     for (int off = LPR / 2; off >= 1; off >>= 1) acc += __shfl_xor(acc, off);
     if (seg == 0) rv[RVEC + r] = acc;
   };
-  // Tiles whose every query row precedes every key row are skipped (dS = 0, nothing stored).
-  auto live = [&](int ii0) { return ii0 < T && !(CAUSAL && ii0 + 31 < j0); };
+  // Tiles whose every query row precedes every key row, or without a key row, are skipped (dS = 0,
+  // nothing stored).
+  auto live = [&](int ii0) { return j0 < T && !(CAUSAL && ii0 + 31 < j0); };
   // S (query rows ii0 + R(r, half), key my_j) -> P = e^{S - L}; masked entries and key rows past
   // T give exactly 0.
   auto probabilities = [&](f32x16& sacc, int ii0, const float* ls) {
@@ -643,7 +645,7 @@ __global__ __launch_bounds__(256, kDkdvMinWaves<HS>) void fa2_bwd_dkdv_kernel(
     probabilities(sacc, ii0, rv);
     accumulate(dvacc, images + 3 * IMAGE, sacc);
     score_gradients(sacc, pacc, rv + RVEC);
-    if (wave_stores) store_ds(pacc, ii0);
+    if (STORE_DS) store_ds(pacc, ii0);
     accumulate(dkacc, images + 2 * IMAGE, pacc);
   }
 
@@ -695,7 +697,7 @@ __global__ __launch_bounds__(256, kDkdvMinWaves<HS>) void fa2_bwd_dkdv_kernel(
       }
       probabilities(sacc, ii0, rv);
       score_gradients(sacc, pacc, rv + RVEC);
-      if (wave_stores) store_ds(pacc, ii0);
+      if (STORE_DS) store_ds(pacc, ii0);
 #pragma unroll
       for (int d = 0; d < HS / 32; ++d)
 #pragma unroll
@@ -777,10 +779,15 @@ __global__ __launch_bounds__(256) void fa2_bwd_dq_sum_kernel(float* __restrict__
 
 // ------------------------------------------------------------------------------------
 // dQ from stored dS tiles: dQ^T += K^T dS^T, one 32x32 tile per MFMA chain.  Workgroup =
-// 32 * WAVES query rows (WAVES = 4, or 2 for short causal heads).  K tiles of 64 rows go
-// global -> registers -> LDS, double
+// 32 * WAVES query rows (WAVES = 4, or 2 for short causal heads).  The product runs on the BF16
+// matrix pipe, six products of three-part operands (split_bf16.hpp; 768 matrix cycles a tile at
+// hs 64, 2048 on the FP32 MFMA).  K stages go global -> registers -> split -> LDS, double
 // buffered; each wave streams its own dS tiles from the workspace straight into registers,
-// one stage ahead, as the B operand.  Heads [bh_base, bh_base + BH).
+// one stage ahead, and splits them there as the B operand.  What bounds it is the read of dS: B1 H32 N8192 D64
+// 2.29 -> 1.58 ms (5.6 TB/s), B4 H32 N4096 causal 1.26 -> 0.91 ms.
+// A stage is 64 keys, or 32 where two buffers of 64 would hold the CU to fewer than three
+// workgroups of four waves (hs 128; two-wave workgroups).  Heads [bh_base, bh_base + BH).
+// Sums that the parts cannot vouch for (split_suspect) run the pass again on FP32 MFMAs.
 // SPLIT (small grids, heads from 0): each item's key stages (pass 0's, then pass 1's) are
 // split over two workgroups, neighbours in the XCD order; part 0 writes dQ, part 1 its
 // partial dQ densely into part_ws, and fa2_bwd_dq_sum_kernel adds the two in that order.
@@ -793,16 +800,20 @@ __global__ __launch_bounds__(64 * WAVES, 2) void fa2_bwd_dq_ds_kernel(
     const float* __restrict__ K, const float* __restrict__ dsw, float* __restrict__ dQ, int nh,
     int T, int bh_base, int BH, int n_qtiles, RowStrides sk, RowStrides sdq, float scale,
     float* __restrict__ part_ws = nullptr, int heads_per_xcd = 0) {
-  constexpr int BN = 64;
+  constexpr int BN = HS == 128 || WAVES == 2 ? 32 : 64;
   constexpr int NSUB = BN / 32;
   constexpr int THREADS = 64 * WAVES;
   constexpr int BM = 32 * WAVES;  // query rows per workgroup, 32 per wave
-  constexpr int KP = HS + 8;  // column reads of rows R(kk, 0) and R(kk, 1) = +4: disjoint banks
-  constexpr int TILE = BN * KP;
-  constexpr int F4_ROW = HS / 4;
-  constexpr int LOADS = BN * F4_ROW / THREADS;
-  static_assert(BN * F4_ROW % THREADS == 0, "tile must split evenly over the workgroup");
-  __shared__ __attribute__((aligned(16))) float smem[2 * TILE];
+  // LDS image of a K stage in units of eight values of one part (16 bytes): unit (sub, d, sh) =
+  // the eight keys of sub's that half sh & 1 takes in step sh >> 1 (16 st + 4 half + 0..3 and
+  // + 8..11: the keys of a lane's two dS float4), at (sub, d/32, sh, d % 32).
+  constexpr int PART = BN * HS * 2;
+  constexpr int STAGE = 3 * PART;
+  constexpr int NU = BN * HS / 8 / THREADS;
+  static_assert(BN * HS / 8 % THREADS == 0, "units must split evenly over the workgroup");
+  constexpr int KP = HS + 8;  // row pitch of the FP32 stage (second run)
+  static_assert(BN * KP * 4 <= 2 * STAGE, "the FP32 stage fits");
+  __shared__ __attribute__((aligned(16))) char smem[2 * STAGE];
 
   const int tid = threadIdx.x;
   const int lane = tid & 63, wave = wave_index();
@@ -868,27 +879,38 @@ __global__ __launch_bounds__(64 * WAVES, 2) void fa2_bwd_dq_ds_kernel(
   // nothing).  The compiler can then
   // count the loads in flight exactly: the MFMAs of stage s wait only for stage s's dS, not
   // for the stage s+1 loads issued ahead of them.
-  float4 kst[LOADS];
+  float kst[NU][8];
   // K rows through a buffer resource over the stage's valid rows (none for a padded stage):
   // keys past T read as zero, as they must, since they meet finite dS columns.
   auto gload = [&](int stage) {
     const int j0 = stage * BN;
     const int rows = min(BN, T - j0);
     const __amdgpu_buffer_rsrc_t rk = rows_rsrc(Kb + (int64_t)j0 * sk.t, rows, sk.t, HS);
+    const int st = (int)sk.t * 4;
 #pragma unroll
-    for (int u = 0; u < LOADS; ++u) {
+    for (int u = 0; u < NU; ++u) {
       const int f = tid + THREADS * u;
-      const int r = f / F4_ROW, c4 = f % F4_ROW;
-      kst[u] = ld4_buffer(rk, (r * (int)sk.t + 4 * c4) * 4);
+      const int d = f % HS, sh = f / HS;  // sh: over the stage's 16-key steps and halves
+      const int at = (16 * (sh >> 1) + 4 * (sh & 1)) * st + 4 * d;
+#pragma unroll
+      for (int j = 0; j < 8; ++j)
+        kst[u][j] = __uint_as_float(__builtin_amdgcn_raw_buffer_load_b32(
+            rk, at, (8 * (j >> 2) + (j & 3)) * st, 0));
     }
   };
   auto lstore = [&](int buf) {
-    float* ks = smem + buf * TILE;
+    char* ks = smem + buf * STAGE;
 #pragma unroll
-    for (int u = 0; u < LOADS; ++u) {
+    for (int u = 0; u < NU; ++u) {
       const int f = tid + THREADS * u;
-      const int r = f / F4_ROW, c4 = f % F4_ROW;
-      st4(ks + r * KP + 4 * c4, kst[u]);
+      const int d = f % HS, sh = f / HS;
+      bf16x8 p[3];
+      split_bf16(kst[u], p);
+#pragma unroll
+      for (int q = 0; q < 3; ++q)
+        *reinterpret_cast<bf16x8*>(
+            ks + q * PART +
+            (((sh >> 2) * (HS / 32) + (d >> 5)) * 128 + (sh & 3) * 32 + (d & 31)) * 16) = p[q];
     }
   };
   // A stored tile exists for query block ib and key block jb iff both lie inside the head and,
@@ -908,21 +930,34 @@ __global__ __launch_bounds__(64 * WAVES, 2) void fa2_bwd_dq_ds_kernel(
       }
     }
   };
-  auto compute = [&](int stage, const float* ks, const float4 (&dr)[NSUB][4]) {
+  auto compute = [&](int stage, const char* ks, const float4 (&dr)[NSUB][4]) {
     if (stage >= s_end) return;  // a padded stage (or, split, the other part's)
 #pragma unroll
     for (int sub = 0; sub < NSUB; ++sub) {
       if (!has_tile(stage * NSUB + sub)) continue;
-      // kk-major: the HS/32 accumulator chains alternate, so no MFMA waits on its predecessor
-      // K^T operand (key row R(kk, half), column d*32 + col): lane base pointer plus
-      // compile-time row offsets, carried by the LDS reads as immediates.
-      const float* kcol = ks + (sub * 32 + 4 * half) * KP + col;
 #pragma unroll
-      for (int kk = 0; kk < 16; ++kk) {
+      for (int st = 0; st < 2; ++st) {
+        const float4 lo = dr[sub][2 * st], hi = dr[sub][2 * st + 1];
+        const float x[8] = {lo.x, lo.y, lo.z, lo.w, hi.x, hi.y, hi.z, hi.w};
+        bf16x8 dp[3];
+        split_bf16(x, dp);
 #pragma unroll
-        for (int d = 0; d < HS / 32; ++d)
-          acc[d] = mfma32(kcol[(8 * (kk >> 2) + (kk & 3)) * KP + d * 32],
-                          f4_at(dr[sub][kk >> 2], kk & 3), acc[d]);
+        for (int d0 = 0; d0 < HS / 32; d0 += 2) {
+          constexpr int ND = HS / 32 < 2 ? 1 : 2;  // two chains
+          bf16x8 a[ND][3];
+#pragma unroll
+          for (int d = 0; d < ND; ++d)
+#pragma unroll
+            for (int q = 2; q >= 0; --q)
+              a[d][q] = *reinterpret_cast<const bf16x8*>(
+                  ks + q * PART +
+                  ((sub * (HS / 32) + d0 + d) * 128 + (2 * st + half) * 32 + col) * 16);
+#pragma unroll
+          for (int p = 0; p < 6; ++p)
+#pragma unroll
+            for (int d = 0; d < ND; ++d)
+              acc[d0 + d] = mfma_bf16(a[d][kSplitA[p]], dp[kSplitB[p]], acc[d0 + d]);
+        }
       }
     }
   };
@@ -930,7 +965,7 @@ __global__ __launch_bounds__(64 * WAVES, 2) void fa2_bwd_dq_ds_kernel(
     const int buf = (s - s_begin) & 1;
     gload(s + 1);
     dsload(s + 1, nxt);
-    compute(s, smem + buf * TILE, cur);
+    compute(s, smem + buf * STAGE, cur);
     lstore(buf ^ 1);
     __syncthreads();
   };
@@ -949,6 +984,37 @@ __global__ __launch_bounds__(64 * WAVES, 2) void fa2_bwd_dq_ds_kernel(
     }
   }
 
+  bool odd = false;
+#pragma unroll
+  for (int d = 0; d < HS / 32; ++d) odd |= split_suspect(acc[d]);
+  if (__syncthreads_or(odd)) {
+    float* const ks = reinterpret_cast<float*>(smem);
+#pragma unroll
+    for (int d = 0; d < HS / 32; ++d) acc[d] = zero16();
+    for (int s = s_begin; s < s_end; ++s) {
+      __syncthreads();
+      for (int f = tid; f < BN * HS / 4; f += THREADS) {
+        const int r = f / (HS / 4), c4 = f % (HS / 4) * 4;
+        const int64_t j = (int64_t)s * BN + r;
+        st4(ks + r * KP + c4, j < T ? ld4(Kb + j * sk.t + c4) : zero4());
+      }
+      __syncthreads();
+      float4 dr[NSUB][4];
+      dsload(s, dr);
+#pragma unroll
+      for (int sub = 0; sub < NSUB; ++sub) {
+        if (!has_tile(s * NSUB + sub)) continue;
+#pragma unroll
+        for (int kk = 0; kk < 16; ++kk)
+#pragma unroll
+          for (int d = 0; d < HS / 32; ++d)
+            acc[d] = mfma32(ks[(sub * 32 + mfma_row(kk, half)) * KP + d * 32 + col],
+                            f4_at(dr[sub][kk >> 2], kk & 3), acc[d]);
+      }
+    }
+    __syncthreads();
+  }
+
   if (my_i < T) {
     float* op = dQ + b * sdq.b + h * sdq.h + (int64_t)my_i * sdq.t;
     if (SPLIT && part) op = part_ws + ((int64_t)bh * T + my_i) * HS;
@@ -962,7 +1028,7 @@ __global__ __launch_bounds__(64 * WAVES, 2) void fa2_bwd_dq_ds_kernel(
       }
     }
   }
-  }  // pass: the stage loop ended on a barrier, so the next pass may refill LDS
+  }  // pass: the check above is a barrier, so the next pass may refill LDS
 }
 
 RowStrides rs(const int64_t* s) { return RowStrides{s[0], s[1], s[2]}; }
