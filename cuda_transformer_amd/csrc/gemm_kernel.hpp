@@ -25,23 +25,26 @@
 // 5.0e-7; K = 8192: 5.7e-7 against 1.6e-6).
 // Sustained on all CUs, from registers, the six products reach 305 TFLOP/s of FP32 work (the
 // chip's power limit), the FP32 MFMA 154.
-// What three bfloat16 numbers cannot hold: infinities, values that round to one (above 3.39e38),
-// and the low bits of magnitudes below 2^-109.  A workgroup whose tile of sums comes out with a
-// value that is not finite, or is nonzero below 2^-100, discards it and runs the tile again with
-// FP32 MFMAs (exact_tile), so such operands give what FP32 arithmetic gives.
+// Operands are scaled by 2^24 before the split (split_bf16.hpp), so that the parts hold every float
+// below 2^103 exactly, subnormals included, and products keep their bits down to where FP32's own
+// end.  Sums above 2^79 overflow, infinities and larger operands give NaN: a workgroup whose tile
+// comes out with a value that is not finite discards it and runs the tile again with FP32 MFMAs
+// (exact_tile), so such operands give what FP32 arithmetic gives, in up to 2.4 times the time
+// (8192 x 3072 x 768 with an infinity in every tile: 212 -> 516 us).
 //
 // gfx950 design: workgroup tile 128x128 of four 64x64 waves, 64x128 of four 32x64 or 64x64 of
-// four 32x32, two or three workgroups (waves per SIMD) on a CU.  A lane loads eight k of one row (two dwordx4
-// where k is contiguous in memory, eight coalesced dwords where the rows are), splits them
-// (11 VALU instructions per pair, beside the MFMAs) and stores one 16-byte unit per
+// four 32x32, two or three workgroups (waves per SIMD) on a CU.  A lane loads eight k of one row
+// (two dwordx4 where k is contiguous in memory, eight dwords otherwise), scales and splits them
+// (13 VALU instructions per pair, beside the MFMAs) and stores one 16-byte unit per
 // part: LDS holds [part][k half][row][8 k], which is the MFMA operand order, so operand reads
 // and stores are contiguous 16-byte accesses with no bank conflict and no padding to speak of.
 // Loads and the epilogue's stores go through buffer resources: scalar bases with fixed per-lane
 // offsets, and the buffer's range check zeroes (loads) or drops (stores) what lies outside the
 // operand, so the K loop and the epilogue carry no per-element address arithmetic or bounds
-// tests.  What bounds it: 8192 x 3072 x 768 runs at 185 TFLOP/s (FP32 MFMA: 142) with the matrix
-// pipe 54% busy at 1.93 GHz, the chip's power limit (on all-zero operands the same kernel clocks
-// 2.45 GHz and takes 167 us instead of 209), so bytes moved per product cost time too.
+// tests.  What bounds it: 8192 x 3072 x 768 runs at 182 TFLOP/s (FP32 MFMA: 142; without the scale
+// 185, with the matrix pipe 54% busy at 1.93 GHz), at the chip's power limit (on all-zero operands
+// the same kernel clocks 2.45 GHz and takes 167 us instead of 209), so bytes moved per product and
+// the splits' instructions cost time too.
 //
 // This header holds the kernel templates and the per-tile launcher; gemm_tiles_*.hip each
 // instantiate a few tile types (gemm_launch_<tile>), so the build compiles them in parallel, and
@@ -212,7 +215,7 @@ __device__ __forceinline__ void store_slice(const Slice<ROWS, THREADS>& L, char*
     int r, h;
     unit_coords<MODE, ROWS>(f, r, h);
     bf16x8 p[3];
-    split_bf16(L.v[u], p);
+    split_bf16<true>(L.v[u], p);
     char* at = lds + h * (PLANE / 2) + r * 16;
 #pragma unroll
     for (int q = 0; q < 3; ++q) *reinterpret_cast<bf16x8*>(at + q * PLANE) = p[q];
@@ -388,7 +391,7 @@ __device__ __forceinline__ void block_store(const f32x16 (&acc)[TL::MB][TL::NB],
   }
 }
 
-// The tile's sums with FP32 MFMAs, for operands that three bfloat16 parts cannot hold: the same
+// The tile's sums with FP32 MFMAs, for operands or sums that the parts cannot hold: the same
 // loads, FP32 slices in LDS as [k][row], one buffer.  Every thread of the workgroup calls it.
 template <class TL, class PA, class PB>
 __device__ __forceinline__ void exact_tile(const PA& pa, const PB& pb, typename PA::S& la,
@@ -566,14 +569,15 @@ __global__ __launch_bounds__(TL::THREADS, 2) void gemm_kernel(GemmOperand A, Gem
     slice(f1, f0, la1, lb1, la0, lb0, buf0, t + 3);
   }
 
-  // Sums that the split cannot vouch for (see the top): the whole workgroup runs the tile again.
+  // Sums that are not finite (see the top): the whole workgroup runs the tile again.
   bool odd = false;
 #pragma unroll
   for (int i = 0; i < MB; ++i)
 #pragma unroll
     for (int j = 0; j < NB; ++j) {
       acc[i][j] += low[i][j];
-      odd |= split_suspect(acc[i][j]);
+      odd |= not_finite(acc[i][j]);
+      acc[i][j] *= kSplitUnscale * kSplitUnscale;
     }
   if (__syncthreads_or(odd))
     exact_tile<TL>(pa, pb, la0, lb0, reinterpret_cast<float*>(smem), nk, tid, wm, wn, half, col,

@@ -70,3 +70,88 @@ def test_gemm_outside_the_split_range(cuda, m, k, n):
     bound = _bound(x, w)
     rows = [i for i in range(m) if i not in (3, 4, 5, 6)]
     assert torch.all((out.double() - ref).abs()[rows] <= bound[rows] + 1e-45)
+
+
+# Powers of two on the operands: products of ordinary size of one tiny and one large operand, down
+# to subnormal x, and up to sums near the top of the range.
+SCALES = [(-60, 60), (-100, 20), (-109, 60), (-116, 60), (-120, 40), (-126, 100), (-130, 60),
+          (-136, 60), (-136, 20), (-140, 120), (-70, -70), (60, 60), (100, -130), (2, -148)]
+
+
+@pytest.mark.parametrize("a,b", SCALES)
+@pytest.mark.parametrize("m,k,n,order", [(70, 768, 66, "nn"), (300, 40, 2000, "tn"),
+                                         (130, 2048, 130, "nt"), (33, 70, 40, "sn")])
+def test_gemm_scaled_operands(cuda, m, k, n, order, a, b):
+    """Every finite operand takes part with all of its bits, whatever its magnitude and its
+    partner's: the bound of ordinary operands, plus FP32's subnormal spacing a step."""
+    from cuda_transformer.ops import cuda_fma
+
+    x, w, xc, wc = _operands(m, k, n, order, m + k)
+    for t in (x, xc):
+        t *= 2.0 ** a
+    for t in (w, wc):
+        t *= 2.0 ** b
+    x, w = xc[0].cpu().contiguous(), wc.cpu().contiguous()  # as rounded to FP32
+    out = cuda_fma(xc, wc, torch.zeros(n, device=cuda))[0].double().cpu()
+    assert torch.all((out - x.double() @ w.double()).abs() <= _bound(x, w) + k * 2.0 ** -149)
+
+
+@pytest.mark.parametrize("order", ["nn", "nt", "tn", "tt", "sn", "ns"])
+def test_gemm_scales_that_cancel(cuda, order):
+    """Column k of x times 2^-e, row k of w times 2^e, e = 124 and -124 in turn: every product is of
+    ordinary size, and the result the unscaled operands'."""
+    from cuda_transformer.ops import cuda_fma
+
+    m, k, n = 130, 300, 140
+    x, w, xc, wc = _operands(m, k, n, order, 17)
+    e = torch.tensor([124.0, -124.0]).repeat(k // 2)
+    xc *= (2.0 ** -e.double()).float().to(cuda)
+    wc *= (2.0 ** e.double()).float().to(cuda)[:, None]
+    out = cuda_fma(xc, wc, torch.zeros(n, device=cuda))[0].double().cpu()
+    assert torch.all((out - x.double() @ w.double()).abs() <= _bound(x, w))
+
+
+@pytest.mark.parametrize("order", ["nn", "nt", "tn", "tt", "sn", "ns"])
+def test_gemm_second_run_orders(cuda, order):
+    """A tile that runs again on FP32 MFMAs (an infinity in one row), in each load order."""
+    from cuda_transformer.ops import cuda_fma
+
+    m, k, n = 200, 77, 133
+    x, w, xc, wc = _operands(m, k, n, order, 23)
+    w, wc = w.abs() + 0.5, wc.abs() + 0.5
+    xc[0, 3, 5] = float("inf")
+    out = cuda_fma(xc, wc, torch.zeros(n, device=cuda))[0].double().cpu()
+    assert torch.all(out[3] == float("inf"))
+    rows = [i for i in range(m) if i != 3]
+    assert torch.all((out - x.double() @ w.double()).abs()[rows] <= _bound(x, w)[rows])
+
+
+@pytest.mark.parametrize("rows,k,n", [(300, 70, 65), (3000, 96, 132), (129, 33, 1155)])
+def test_weight_bias_grad_second_run(cuda, rows, k, n):
+    """dW tiles that run again on FP32 MFMAs beside the column sums that share their LDS, at odd
+    and even n, split along the rows and not: dW and db as without the infinity elsewhere."""
+    from cuda_transformer_amd.ops import linear_weight_bias_grad
+
+    g = torch.Generator().manual_seed(rows + n)
+    x, dy = torch.randn(rows, k, generator=g), torch.randn(rows, n, generator=g)
+    x[7, 3] = float("inf")
+    dy[7] = dy[7].abs() + 0.5
+    dw, db = (t.double().cpu() for t in linear_weight_bias_grad(x.to(cuda), dy.to(cuda)))
+    assert torch.all(dw[3] == float("inf"))
+    x[:, 3] = 0.0
+    dw[3] = 0.0
+    assert torch.all((dw - x.double().t() @ dy.double()).abs() <= _bound(x.t(), dy))
+    assert torch.all((db - dy.double().sum(0)).abs() <= 1e-6 * dy.double().abs().sum(0))
+
+
+def test_weight_bias_grad_column_strides(cuda):
+    """dy with strided columns: db from the column-sum kernels, not the GEMM's slices."""
+    from cuda_transformer_amd.ops import linear_weight_bias_grad
+
+    g = torch.Generator().manual_seed(9)
+    x, dy = torch.randn(500, 40, generator=g), torch.randn(500, 50, generator=g)
+    wide = torch.zeros(500, 50, 2)
+    wide[..., 0] = dy
+    dw, db = (t.double().cpu() for t in linear_weight_bias_grad(x.to(cuda), wide.to(cuda)[..., 0]))
+    assert torch.all((dw - x.double().t() @ dy.double()).abs() <= _bound(x.t(), dy))
+    assert torch.all((db - dy.double().sum(0)).abs() <= 1e-6 * dy.double().abs().sum(0))
