@@ -59,8 +59,9 @@ namespace cta {
 
 // How an operand's slices are loaded: k contiguous with rows a multiple of 16 bytes apart
 // (kVecK), k contiguous with any row stride or length (kAnyK), rows contiguous (kVecMN: m of A,
-// n of B; any alignment), or any strides at all (kScalar, only ever for both operands).
-enum LoadMode { kVecK = 0, kVecMN = 1, kScalar = 2, kAnyK = 3 };
+// n of B; any alignment), any strides whose slices 32-bit offsets reach (kStrided), or any strides
+// at all (kScalar, only ever for both operands).
+enum LoadMode { kVecK = 0, kVecMN = 1, kScalar = 2, kAnyK = 3, kStrided = 4 };
 
 namespace {
 
@@ -108,7 +109,10 @@ __device__ __forceinline__ void unit_coords(int f, int& r, int& h) {
 // zero (kVecK, kAnyK) or in-bounds values that only feed output rows/columns never stored
 // (kVecMN).  On a ragged last slice a kVecK lane whose k lies past the end moves its offset out
 // of range; kAnyK, whose end may fall inside a lane's four k, loads that slice by single dwords
-// (its whole slices are dwordx4 loads too: buffer loads need only 4-byte alignment).
+// (its whole slices are dwordx4 loads too: buffer loads need only 4-byte alignment).  kStrided
+// loads every slice by single dwords, rows past the end moved out of range, and zeroes k past the
+// end in registers (2048 x 3072 x 768 with every second column of a wider x: 107 us, 132 with
+// kScalar loads of both operands; with every second column of a wider W 70 and 134).
 template <int MODE, int ROWS, int THREADS>
 struct LoadPlan {
   using S = Slice<ROWS, THREADS>;
@@ -118,12 +122,12 @@ struct LoadPlan {
   int rows;           // valid rows from row0: min(ROWS, R - row0) (kVecK) or R - row0 (kVecMN)
   int row0, kb, R, ke;
   int voff[N];        // vector modes: byte offset of the lane's unit within a slice
-  int kq;             // kVecK, kAnyK: the unit's first k within a slice (the same for all its units)
+  int kq;             // not kVecMN: the unit's first k within a slice (the same for all its units)
   __device__ __forceinline__ void init(const float* b, int64_t sr, int64_t sk, int r0, int k0,
                                        int R_, int K_, int tid) {
     s_row = sr; s_k = sk; row0 = r0; kb = k0; R = R_; ke = K_;
-    if (MODE == kVecK || MODE == kAnyK) {
-      base = b + (int64_t)r0 * sr + k0;
+    if (MODE == kVecK || MODE == kAnyK || MODE == kStrided) {
+      base = b + (int64_t)r0 * sr + (int64_t)k0 * (MODE == kStrided ? sk : 1);
       rows = min(ROWS, R_ - r0);
     } else if (MODE == kVecMN) {
       base = b + (int64_t)k0 * sk + r0;
@@ -137,9 +141,10 @@ struct LoadPlan {
       const int f = tid + THREADS * u;
       int r, h;
       unit_coords<MODE, ROWS>(f, r, h);
-      voff[u] = MODE == kVecMN ? (int)(((int64_t)(8 * h) * sk + r) * 4)
-                               : (int)(((int64_t)r * sr + 8 * h) * 4);
-      if (f >= S::UNITS) voff[u] = (int)0x80000000;
+      voff[u] = MODE == kVecMN     ? (int)(((int64_t)(8 * h) * sk + r) * 4)
+                : MODE == kStrided ? (int)(((int64_t)r * sr + 8 * h * sk) * 4)
+                                   : (int)(((int64_t)r * sr + 8 * h) * 4);
+      if (f >= S::UNITS || (MODE == kStrided && r >= rows)) voff[u] = (int)0x80000000;
     }
   }
   static __device__ __forceinline__ void coords(int f, int& r, int& h) {
@@ -163,15 +168,14 @@ struct LoadPlan {
       }
       return;
     }
-    const float* bt;
-    int nbytes;
-    if (MODE == kVecK || MODE == kAnyK) {
-      bt = base + (int64_t)t * kGemmK;
-      nbytes = klim > 0 ? (int)(((int64_t)(rows - 1) * s_row + klim) * 4) : 0;
-    } else {
-      bt = base + (int64_t)t * kGemmK * s_k;
-      nbytes = klim > 0 ? (int)(((int64_t)(klim - 1) * s_k + rows) * 4) : 0;
-    }
+    // 32 bits reach (pick_mode), and the product by 0 or 1 stays scalar arithmetic: a conditional
+    // becomes a branch that splits the K loop's schedule (64 more VGPRs where both operands load
+    // dwords, scratch in some kStrided kernels).
+    const float* bt = base + (int64_t)t * kGemmK * (MODE == kVecK || MODE == kAnyK ? 1 : s_k);
+    const int last = MODE == kVecK || MODE == kAnyK ? (rows - 1) * (int)s_row + klim
+                     : MODE == kVecMN               ? (klim - 1) * (int)s_k + rows
+                                      : (rows - 1) * (int)s_row + (klim - 1) * (int)s_k + 1;
+    const int nbytes = last * 4 * min(max(klim, 0), 1);
     const __amdgpu_buffer_rsrc_t rs =
         __builtin_amdgcn_make_buffer_rsrc(const_cast<float*>(bt), (short)0, nbytes, 0x00020000);
     if (MODE == kAnyK && klim < kGemmK) {  // uniform
@@ -200,6 +204,16 @@ struct LoadPlan {
           L.v[u][e] = __uint_as_float(
               __builtin_amdgcn_raw_buffer_load_b32(rs, voff[u], e * kbytes, 0));
       }
+    }
+  }
+  // kStrided: what slice t, in registers, holds past the end of K (other elements of the operand).
+  __device__ __forceinline__ void mask(S& L, int t) const {
+    if constexpr (MODE == kStrided) {
+      const int klim = ke - (kb + t * kGemmK) - kq;
+#pragma unroll
+      for (int u = 0; u < N; ++u)
+#pragma unroll
+        for (int e = 0; e < 8; ++e) L.v[u][e] = e < klim ? L.v[u][e] : 0.0f;
     }
   }
 };
@@ -420,6 +434,8 @@ __device__ __forceinline__ void exact_tile(const PA& pa, const PB& pb, typename 
   for (int t = 0; t < nk; ++t) {
     pa.load(la, t, tid);
     pb.load(lb, t, tid);
+    pa.mask(la, t);
+    pb.mask(lb, t);
     __syncthreads();
     put(pa, la, as, BM);
     put(pb, lb, bs, BN);
@@ -537,6 +553,8 @@ __global__ __launch_bounds__(TL::THREADS, 2) void gemm_kernel(GemmOperand A, Gem
   pb.load(lb0, 0, tid);
   pa.load(la1, 1, tid);
   pb.load(lb1, 1, tid);
+  pa.mask(la0, 0);
+  pb.mask(lb0, 0);
   store_slice<AMODE, BM, THREADS, PA>(la0, buf0, tid);
   store_slice<BMODE, BN, THREADS, PB>(lb0, buf0 + TL::A_BYTES, tid);
   add_cs(lb0);
@@ -551,11 +569,13 @@ __global__ __launch_bounds__(TL::THREADS, 2) void gemm_kernel(GemmOperand A, Gem
   Frags<TL> f0, f1;
   read_frags<TL>(buf0, f0, wm, wn, half, col);
   auto slice = [&](Frags<TL>& cur, Frags<TL>& nxt, typename PlanA::S& la_far,
-                   typename PlanB::S& lb_far, const typename PlanA::S& la_next,
-                   const typename PlanB::S& lb_next, char* nbuf, int t_far) {
+                   typename PlanB::S& lb_far, typename PlanA::S& la_next,
+                   typename PlanB::S& lb_next, char* nbuf, int t_far) {
     pa.load(la_far, t_far, tid);
     pb.load(lb_far, t_far, tid);
     mma_products<TL, 0, 3>(cur, acc, low);
+    pa.mask(la_next, t_far - 1);
+    pb.mask(lb_next, t_far - 1);
     store_slice<AMODE, BM, THREADS, PA>(la_next, nbuf, tid);
     store_slice<BMODE, BN, THREADS, PB>(lb_next, nbuf + TL::A_BYTES, tid);
     add_cs(lb_next);
@@ -691,6 +711,7 @@ int pick_mode(const GemmOperand& op, bool is_a, int64_t rows, int64_t K) {
   if (s_mn == 1 && rows >= 1 && s_k >= rows &&
       (63 * s_k + std::max<int64_t>(rows, 256)) * 4 < kMaxBytes)
     return kVecMN;
+  if (s_k >= 0 && s_mn >= 0 && (127 * s_mn + 15 * s_k + 1) * 4 < kMaxBytes) return kStrided;
   return kScalar;
 }
 
@@ -709,6 +730,9 @@ void dispatch_b(int bm, dim3 grid, hipStream_t st, const GemmOperand& A, const G
                        zin, Z, kchunk, ws);
   else if (bm == kAnyK)
     hipLaunchKernelGGL((gemm_kernel<TL, AM, kAnyK>), grid, block, 0, st, A, B, C, ep, M, N, K,
+                       zin, Z, kchunk, ws);
+  else if (bm == kStrided)
+    hipLaunchKernelGGL((gemm_kernel<TL, AM, kStrided>), grid, block, 0, st, A, B, C, ep, M, N, K,
                        zin, Z, kchunk, ws);
   else
     hipLaunchKernelGGL((gemm_kernel<TL, AM, kVecMN>), grid, block, 0, st, A, B, C, ep, M, N, K,
@@ -729,6 +753,8 @@ void dispatch_a(int am, int bm, dim3 grid, hipStream_t st, const GemmOperand& A,
     dispatch_b<TL, kVecK, CS>(bm, grid, st, A, B, C, ep, M, N, K, zin, Z, kchunk, ws);
   else if (am == kAnyK)
     dispatch_b<TL, kAnyK, CS>(bm, grid, st, A, B, C, ep, M, N, K, zin, Z, kchunk, ws);
+  else if (am == kStrided)
+    dispatch_b<TL, kStrided, CS>(bm, grid, st, A, B, C, ep, M, N, K, zin, Z, kchunk, ws);
   else if (am == kVecMN)
     dispatch_b<TL, kVecMN, CS>(bm, grid, st, A, B, C, ep, M, N, K, zin, Z, kchunk, ws);
   else if constexpr (CS)
