@@ -22,9 +22,11 @@
 //  * O^T = V^T P^T takes the score registers, split in place, as the B operand: registers
 //    8s .. 8s + 7 are step s's eight keys of this lane's half, and V's image holds its keys in
 //    that order.  P never leaves registers.
-//  * A pass whose sums are not finite, or nonzero below 2^-100, is run again on FP32 MFMAs by
-//    the whole workgroup, so infinities, NaN and the ends of FP32's range give what FP32
-//    arithmetic gives.
+//  * Q, P and V are scaled by 2^24 before they are split, so their parts hold every bit of them
+//    (split_bf16.hpp); K's may lack what lies below 2^-133, which moves no score that matters
+//    while |q| < 2^85 (kMaxScoreFactor).  A pass with a larger q, or whose sums are not finite, is run again on
+//    FP32 MFMAs by the whole workgroup, so infinities, NaN and values up to FP32's largest give
+//    what FP32 arithmetic gives.
 //  * Exponentials use exp2 with log2(e) folded into the scale; L is exported in natural log.
 //  * Lazy rescaling: the running max m used as the exponent offset only moves when some row
 //    of the wave sees a tile max more than 2^8 above it (a wave-uniform vote).  Otherwise the
@@ -57,7 +59,8 @@ template <> struct FwdTile<128> { static constexpr int BN = 32; static constexpr
 
 // One online-softmax step of a wave's 32x32 score tile (lane: 16 scores of its query row): the
 // mask, the lazily moved offset m and P = 2^{(S - m) c} in place of S.  `rescale(alpha)` scales
-// the output accumulators when the offset moves.
+// the output accumulators when the offset moves.  S and m may carry a power of two that c and
+// rescale_gap take back.
 template <bool CAUSAL, class F>
 __device__ __forceinline__ void softmax_step(f32x16& sacc, int jj0, int i0, int my_i, int T,
                                              int half, float scale_log2, float rescale_gap,
@@ -176,6 +179,7 @@ __global__ __launch_bounds__(64 * WAVES, FwdTile<HS>::MINW) void fa2_fwd_kernel(
 
   // Q parts of this lane's row, the B operands of the score product: step s, d 16s + 8 half + j.
   bf16x8 qp[HS / 16][3];
+  float qmax = 0.0f;
 #pragma unroll
   for (int st = 0; st < HS / 16; ++st) {
     float x[8];
@@ -185,8 +189,13 @@ __global__ __launch_bounds__(64 * WAVES, FwdTile<HS>::MINW) void fa2_fwd_kernel(
       const float4 v = my_i < T ? ld4(q8 + 4 * c) : zero4();
       x[4 * c] = v.x; x[4 * c + 1] = v.y; x[4 * c + 2] = v.z; x[4 * c + 3] = v.w;
     }
-    split_bf16(x, qp[st]);
+    split_bf16<true>(x, qp[st]);
+#pragma unroll
+    for (int e = 0; e < 8; e += 2) qmax = fmaxf(fmaxf(qmax, fabsf(x[e])), fabsf(x[e + 1]));
   }
+  // The pass runs again on FP32 MFMAs.  (The vote is taken here: left to the end of the pass, it
+  // would keep Q in registers.  A NaN shows in the row's sum.)
+  bool odd = __any(qmax >= kMaxScoreFactor);
 
   // O: the products of the first parts and the smaller ones apart (see gemm_kernel.hpp)
   f32x16 oacc[HS / 32], olow[HS / 32];
@@ -245,7 +254,7 @@ __global__ __launch_bounds__(64 * WAVES, FwdTile<HS>::MINW) void fa2_fwd_kernel(
 #pragma unroll
       for (int q = 0; q < 3; ++q)
         *reinterpret_cast<bf16x8*>(ks + q * PART + (d8 * 32 + (key ^ (d8 & 7))) * 16) = p[q];
-      split_bf16(vst[u], p);
+      split_bf16<true>(vst[u], p);
 #pragma unroll
       for (int q = 0; q < 3; ++q)
         *reinterpret_cast<bf16x8*>(vs + q * PART + ((d >> 5) * 128 + sh * 32 + (d & 31)) * 16) = p[q];
@@ -293,8 +302,8 @@ __global__ __launch_bounds__(64 * WAVES, FwdTile<HS>::MINW) void fa2_fwd_kernel(
         }
       }
       sacc += sodd;
-      softmax_step<CAUSAL>(sacc, jj0, i0, my_i, T, half, scale_log2, rescale_gap, m_run, l_run,
-                           [&](float alpha) {
+      softmax_step<CAUSAL>(sacc, jj0, i0, my_i, T, half, scale_log2 * kSplitUnscale,
+                           rescale_gap * kSplitScale, m_run, l_run, [&](float alpha) {
 #pragma unroll
                              for (int d = 0; d < HS / 32; ++d) { oacc[d] *= alpha; olow[d] *= alpha; }
                            });
@@ -311,7 +320,7 @@ __global__ __launch_bounds__(64 * WAVES, FwdTile<HS>::MINW) void fa2_fwd_kernel(
           for (int q = 2; q >= 0; --q)
             va[d][q] = *reinterpret_cast<const bf16x8*>(
                 vs + q * PART + (d * 128 + (2 * st + half) * 32 + col) * 16);
-        split_bf16(x, pp);
+        split_bf16<true>(x, pp);
 #pragma unroll
         for (int p = 0; p < 6; ++p)
 #pragma unroll
@@ -326,19 +335,21 @@ __global__ __launch_bounds__(64 * WAVES, FwdTile<HS>::MINW) void fa2_fwd_kernel(
     __syncthreads();
   }
 
-  // Sums that the split cannot vouch for (not finite, or nonzero below 2^-100; see
-  // split_bf16.hpp): the workgroup runs the pass again on FP32 MFMAs.
-  bool odd = !(l_run < INFINITY);
+  // Out of the parts' range (see the top): the workgroup runs the pass again on FP32 MFMAs.
+  odd |= !(l_run < INFINITY);
+  m_run *= kSplitUnscale;
+  float o_scale = kSplitScale * kSplitScale;  // of the sums in oacc
 #pragma unroll
   for (int d = 0; d < HS / 32; ++d) {
     oacc[d] += olow[d];
-    odd |= split_suspect(oacc[d]);
+    odd |= not_finite(oacc[d]);
   }
   if (__syncthreads_or(odd)) {
     float* const ks = reinterpret_cast<float*>(smem);
     float* const vs = ks + BN * KP;
     m_run = -INFINITY;
     l_run = 0.0f;
+    o_scale = 1.0f;
 #pragma unroll
     for (int d = 0; d < HS / 32; ++d) oacc[d] = zero16();
     for (int i = i_begin; i < i_end; ++i) {
@@ -378,12 +389,13 @@ __global__ __launch_bounds__(64 * WAVES, FwdTile<HS>::MINW) void fa2_fwd_kernel(
   }
 
   const float l_tot = sum_halves(l_run);
+  const float l_div = l_tot * o_scale;
   if (my_i < T) {
     if constexpr (SPLIT) {
       // A part may have seen no key of this row (l = 0): O = 0, L = -inf, which the merge
       // weighs by e^{-inf} = 0.
       const bool seen = l_tot > 0.0f;
-      const float inv = seen ? 1.0f / l_tot : 0.0f;
+      const float inv = seen ? 1.0f / l_div : 0.0f;
       const int64_t slab = (int64_t)(part - 1) * BH * T;  // part k >= 1: slab k - 1
       float* op = part ? Os + (slab + (int64_t)bh * T + my_i) * HS
                        : O + b * so.b + h * so.h + (int64_t)my_i * so.t;
@@ -406,8 +418,8 @@ __global__ __launch_bounds__(64 * WAVES, FwdTile<HS>::MINW) void fa2_fwd_kernel(
 #pragma unroll
         for (int g = 0; g < 4; ++g) {
           const int dc = d * 32 + 8 * g + 4 * half;
-          st4(op + dc, make_float4(oacc[d][4 * g + 0] / l_tot, oacc[d][4 * g + 1] / l_tot,
-                                   oacc[d][4 * g + 2] / l_tot, oacc[d][4 * g + 3] / l_tot));
+          st4(op + dc, make_float4(oacc[d][4 * g + 0] / l_div, oacc[d][4 * g + 1] / l_div,
+                                   oacc[d][4 * g + 2] / l_div, oacc[d][4 * g + 3] / l_div));
         }
       }
       if (half == 0) L[(int64_t)bh * T + my_i] = m_run * scale + logf(l_tot);

@@ -63,6 +63,11 @@ __device__ __forceinline__ bool not_finite(const f32x16& s) {
   return z != 0.0f;
 }
 
+// Largest magnitude of the scaled operand of the scores whose other operand goes without the scale
+// (q of k in the forward, k of q in the backward): what the other's parts lack, at most 2^-134 an
+// element, moves an exponent by less than 128 x 2^-134 x 2^85 x log2(e) / sqrt(32) < 2^-42.
+constexpr float kMaxScoreFactor = 0x1p85f;
+
 // Whether a sum of split products may differ from FP32 arithmetic by more than rounding: it is
 // infinite or NaN (an operand was, or rounded to infinity), or nonzero below 2^-100 (operands
 // may have been too small for their low parts).  With u = 2 |bits| and T = 2^-100's, the fine

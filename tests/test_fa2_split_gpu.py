@@ -92,3 +92,47 @@ def test_gradients_outside_the_split_range(cuda, T, causal, D):
         assert _rel(x[0, 1], r[0, 1]) <= 1.5e-6
     rows = torch.arange(T) != i
     assert _rel(dq[0, 0, rows], ref[0][0, 0, rows]) <= 1.5e-6
+
+
+@pytest.mark.parametrize("D", [32, 64, 128])
+@pytest.mark.parametrize("T,causal", [(33, True), (160, False), (1100, True)])
+def test_forward_scaled_operands(cuda, T, causal, D):
+    """Scores of a tiny and a large operand, and values of any magnitude, a column each: as
+    accurate as ordinary ones."""
+    from cuda_transformer.ops import flash_attention_fwd
+
+    q, k, v = _qkv(1, 2, T, D, T + D)
+    ref = _ref(q, k, v, causal)
+    for e in (60, 100, 118, 124):
+        for s in (e, -e):
+            o, _ = flash_attention_fwd((q * 2.0 ** -s).to(cuda), (k * 2.0 ** s).to(cuda), v.to(cuda),
+                                       causal)
+            assert _rel(o, ref) <= 1e-6, s
+    e = torch.linspace(-124, 100, D).round()
+    scale = (2.0 ** e.double()).float()
+    o, _ = flash_attention_fwd(q.to(cuda), k.to(cuda), (v * scale).to(cuda), causal)
+    assert _rel(o.cpu().double() / scale.double(), ref) <= 1e-6
+    # subnormal values: FP32's spacing there, and no zeros in their place
+    vs = v.clone()
+    vs[..., 1] *= 2.0 ** -137
+    o, _ = flash_attention_fwd(q.to(cuda), k.to(cuda), vs.to(cuda), causal)
+    assert (o.double().cpu() - _ref(q, k, vs, causal))[..., 1].abs().max() <= 2.0 ** -148
+
+
+@pytest.mark.parametrize("D", [32, 64, 128])
+def test_forward_small_probabilities_of_large_values(cuda, D):
+    """A key of probability 2^-124 holds the only nonzero value of its column, 2^100: the output
+    of 2^-30 has the accuracy of the exponential, whose argument of 124 sees four roundings of at
+    most 2^-24 of it: 4 x 124 x 2^-24 x ln 2 = 2e-5."""
+    from cuda_transformer.ops import flash_attention_fwd
+
+    T = 96
+    q, k, v = _qkv(1, 1, T, D, D)
+    q[..., 0], k[..., 0] = D ** 0.5, 0.0
+    q[..., 1:] = 0.0
+    k[:, :, 5, 0] = -86.0
+    v[..., 2] = 0.0
+    v[:, :, 5, 2] = 2.0 ** 100
+    ref = _ref(q, k, v, False)
+    o, _ = flash_attention_fwd(q.to(cuda), k.to(cuda), v.to(cuda), False)
+    assert _rel(o[..., 2], ref[..., 2]) <= 2e-5
