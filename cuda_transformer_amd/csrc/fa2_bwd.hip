@@ -321,8 +321,12 @@ constexpr int kDsPitch = 40;  // LDS pitch of the per-wave transpose: halves 4 r
 // and dV to dK / dV, part 1 densely to part_ws (dK, then dV, of all BH heads); zeros where a
 // part saw no query stage.  fa2_bwd_dkdv_sum_kernel then adds part 1 to part 0.
 //
-// Sums that the parts cannot vouch for (split_suspect) run the pass again on FP32 MFMAs: a P or
-// dS that is not finite leaves its key's dV or dK not finite, so these two are all that is looked at.
+// k, v, P, dS, and Q and dO but for the rows of Q in S, are scaled before they are split, so the
+// parts hold every bit of them (split_bf16.hpp; Q's rows: kMaxScoreFactor).  Sums that are not
+// finite (infinities, NaN, operands above 2^103, dK or dV above 2^79, dP above 2^79), or |k| above
+// kMaxScoreFactor, run the pass again on FP32 MFMAs: a P or dS that is not finite leaves its key's
+// dV or dK not finite, so these two are all that is looked at.  With every pass run again the
+// backward takes 2.4 to 2.6 times as long.
 template <int HS, bool CAUSAL, bool STORE_DS, bool FOLD, bool SPLIT = false>
 __global__ __launch_bounds__(256, kDkdvMinWaves<HS>) void fa2_bwd_dkdv_kernel(
     const float* __restrict__ Q, const float* __restrict__ K, const float* __restrict__ V,
@@ -417,16 +421,24 @@ __global__ __launch_bounds__(256, kDkdvMinWaves<HS>) void fa2_bwd_dkdv_kernel(
 
   // k's and v's parts, the B operands of S and dP: step st, d 16 st + 8 half + 0..7.
   bf16x8 kp[HS / 16][3], vp[HS / 16][3];
+  float kmax = 0.0f;
 #pragma unroll
   for (int st = 0; st < HS / 16; ++st) {
     auto load = [&](const float* src, bf16x8 (&p)[3]) {
       const float4 x = my_j < T ? ld4(src) : zero4(), y = my_j < T ? ld4(src + 4) : zero4();
       const float v[8] = {x.x, x.y, x.z, x.w, y.x, y.y, y.z, y.w};
-      split_bf16(v, p);
+      split_bf16<true>(v, p);
+      float m = 0.0f;
+#pragma unroll
+      for (int e = 0; e < 8; e += 2) m = fmaxf(fmaxf(m, fabsf(v[e])), fabsf(v[e + 1]));
+      return m;
     };
-    load(Kb + (int64_t)my_j * sk.t + 16 * st + 8 * half, kp[st]);
+    kmax = fmaxf(kmax, load(Kb + (int64_t)my_j * sk.t + 16 * st + 8 * half, kp[st]));
     load(Vb + (int64_t)my_j * sv.t + 16 * st + 8 * half, vp[st]);
   }
+  // The pass runs again on FP32 MFMAs.  (The vote is taken here: left to the end of the pass, it
+  // would keep k in registers.)
+  bool odd = __any(kmax >= kMaxScoreFactor);
 
   f32x16 dkacc[HS / 32], dvacc[HS / 32];
 #pragma unroll
@@ -482,7 +494,8 @@ __global__ __launch_bounds__(256, kDkdvMinWaves<HS>) void fa2_bwd_dkdv_kernel(
         at = (d >> 5) * 128 + sh * 32 + (d & 31);
       }
       bf16x8 p[3];
-      split_bf16(x, p);
+      if (img == 0) split_bf16(x, p);
+      else split_bf16<true>(x, p);
 #pragma unroll
       for (int q = 0; q < 3; ++q)
         *reinterpret_cast<bf16x8*>(images + img * IMAGE + q * PART + at * 16) = p[q];
@@ -513,9 +526,9 @@ __global__ __launch_bounds__(256, kDkdvMinWaves<HS>) void fa2_bwd_dkdv_kernel(
   // Tiles whose every query row precedes every key row, or without a key row, are skipped (dS = 0,
   // nothing stored).
   auto live = [&](int ii0) { return j0 < T && !(CAUSAL && ii0 + 31 < j0); };
-  // S (query rows ii0 + R(r, half), key my_j) -> P = e^{S - L}; masked entries and key rows past
-  // T give exactly 0.
-  auto probabilities = [&](f32x16& sacc, int ii0, const float* ls) {
+  // S (query rows ii0 + R(r, half), key my_j) -> y P, P = e^{S - L} = 2^{S c - L log2(e)}, with
+  // the rows' L log2(e) in ls; masked entries and key rows past T give exactly 0.
+  auto probabilities = [&](f32x16& sacc, int ii0, const float* ls, float c, float y) {
     // A separate block behind a wave-uniform branch: inside the exponential loop the test is
     // if-converted into per-element predication that every tile pays for.
     if ((CAUSAL && ii0 < j0 + 31) || (ii0 + 32 > T) || (j0 + 32 > T)) {
@@ -532,31 +545,34 @@ __global__ __launch_bounds__(256, kDkdvMinWaves<HS>) void fa2_bwd_dkdv_kernel(
       const float lr[4] = {lv.x, lv.y, lv.z, lv.w};
 #pragma unroll
       for (int e = 0; e < 4; ++e)
-        sacc[4 * g + e] = fast_exp2(fmaf(sacc[4 * g + e], scale_log2, -lr[e] * kLog2e));
+        sacc[4 * g + e] = y * fast_exp2(fmaf(sacc[4 * g + e], c, -lr[e]));
     }
   };
-  // dP -> dS = P (dP - delta).  Rounded to FP32 before it is split: fused into the split's first
-  // subtraction (where nothing stores dS) it would give the schedules different bits.
-  auto score_gradients = [&](const f32x16& p, f32x16& pacc, const float* ds) {
+  // dP -> y dS = y P (dP u - delta), y and u powers of two.  Rounded to FP32 before it is split:
+  // fused into the split's first subtraction (where nothing stores dS) it would give the schedules
+  // different bits.
+  auto score_gradients = [&](const f32x16& p, f32x16& pacc, const float* ds, float u) {
 #pragma clang fp contract(off)
 #pragma unroll
     for (int g = 0; g < 4; ++g) {
       const float4 dv = ld4(ds + 8 * g + 4 * half);
       const float dr[4] = {dv.x, dv.y, dv.z, dv.w};
 #pragma unroll
-      for (int e = 0; e < 4; ++e) pacc[4 * g + e] = p[4 * g + e] * (pacc[4 * g + e] - dr[e]);
+      for (int e = 0; e < 4; ++e)
+        pacc[4 * g + e] = p[4 * g + e] * fmaf(pacc[4 * g + e], u, -dr[e]);
     }
   };
   // Lane (col, half) holds dS[ii0 + R(r, half)][j0 + col]: through the wave's transpose buffer
   // as [query][key], 16 queries at a time, and out one query row per lane in whole 256-byte runs.
-  auto store_ds = [&](const f32x16& dsv, int ii0) {
+  // dsv holds dS / u.
+  auto store_ds = [&](const f32x16& dsv, int ii0, float u) {
     float* gt = dsh + ds_tile_index(ii0 / 32, j0 / 32, nb, CAUSAL) * kDsTileFloats;
     const int gs = lane >> 5, hs = (lane >> 4) & 1, c = lane & 15;
 #pragma unroll
     for (int hh = 0; hh < 2; ++hh) {
       wave_lds_fence();
 #pragma unroll
-      for (int r = 0; r < 8; ++r) xpose[mfma_row(r, half) * kDsPitch + col] = dsv[8 * hh + r];
+      for (int r = 0; r < 8; ++r) xpose[mfma_row(r, half) * kDsPitch + col] = dsv[8 * hh + r] * u;
       wave_lds_fence();
 #pragma unroll
       for (int k = 0; k < 2; ++k) {
@@ -582,6 +598,7 @@ __global__ __launch_bounds__(256, kDkdvMinWaves<HS>) void fa2_bwd_dkdv_kernel(
   const bool down = CAUSAL && kt <= n_ktiles - 1 - kt;
   auto stage_at = [&](int i) { return down ? n_stages - 1 - i : q_begin + i; };
   if (i_begin < i_end) issue(stage_at(i_begin), rvec[slot]);
+  constexpr float y = kSplitScale;  // the scale of P and dS in the sums
 
   for (int i = i_begin; i < i_end; ++i) {
     // the stage's copies have landed, and every wave is done with the images
@@ -589,6 +606,7 @@ __global__ __launch_bounds__(256, kDkdvMinWaves<HS>) void fa2_bwd_dkdv_kernel(
     __syncthreads();
     convert();
     float* const rv = rvec[slot];
+    if (tid < BN) rv[tid] *= kLog2e;
     if (FOLD) fold_delta(rv);
     slot ^= 1;
     __syncthreads();
@@ -642,16 +660,19 @@ __global__ __launch_bounds__(256, kDkdvMinWaves<HS>) void fa2_bwd_dkdv_kernel(
         }
       }
     };
-    probabilities(sacc, ii0, rv);
+    probabilities(sacc, ii0, rv, scale_log2 * kSplitUnscale, y);
     accumulate(dvacc, images + 3 * IMAGE, sacc);
-    score_gradients(sacc, pacc, rv + RVEC);
-    if (STORE_DS) store_ds(pacc, ii0);
+    score_gradients(sacc, pacc, rv + RVEC, kSplitUnscale * kSplitUnscale);
+    if (STORE_DS) store_ds(pacc, ii0, y * (kSplitUnscale * kSplitUnscale));
     accumulate(dkacc, images + 2 * IMAGE, pacc);
   }
 
-  bool odd = false;
 #pragma unroll
-  for (int d = 0; d < HS / 32; ++d) odd |= split_suspect(dkacc[d]) || split_suspect(dvacc[d]);
+  for (int d = 0; d < HS / 32; ++d) {
+    odd |= not_finite(dkacc[d]) || not_finite(dvacc[d]);
+    dkacc[d] *= kSplitUnscale * kSplitUnscale;
+    dvacc[d] *= kSplitUnscale * kSplitUnscale;
+  }
   vm_wait_all();  // dS tiles that a second run stores again are stored in order
   if (__syncthreads_or(odd)) {
 #pragma unroll
@@ -669,7 +690,7 @@ __global__ __launch_bounds__(256, kDkdvMinWaves<HS>) void fa2_bwd_dkdv_kernel(
       }
       if (tid < BN) {
         const int64_t t = min(ii0 + tid, T - 1);
-        rv[tid] = Lb[t * sl.t];
+        rv[tid] = Lb[t * sl.t] * kLog2e;
         if (!FOLD) rv[RVEC + tid] = Db[t];
       }
       __syncthreads();
@@ -695,9 +716,9 @@ __global__ __launch_bounds__(256, kDkdvMinWaves<HS>) void fa2_bwd_dkdv_kernel(
         sacc = mfma32(q4.w, k4.w, sacc);
         pacc = mfma32(g4.w, v4.w, pacc);
       }
-      probabilities(sacc, ii0, rv);
-      score_gradients(sacc, pacc, rv + RVEC);
-      if (STORE_DS) store_ds(pacc, ii0);
+      probabilities(sacc, ii0, rv, scale_log2, 1.0f);
+      score_gradients(sacc, pacc, rv + RVEC, 1.0f);
+      if (STORE_DS) store_ds(pacc, ii0, 1.0f);
 #pragma unroll
       for (int d = 0; d < HS / 32; ++d)
 #pragma unroll
@@ -787,7 +808,8 @@ __global__ __launch_bounds__(256) void fa2_bwd_dq_sum_kernel(float* __restrict__
 // 2.29 -> 1.58 ms (5.6 TB/s), B4 H32 N4096 causal 1.26 -> 0.91 ms.
 // A stage is 64 keys, or 32 where two buffers of 64 would hold the CU to fewer than three
 // workgroups of four waves (hs 128; two-wave workgroups).  Heads [bh_base, bh_base + BH).
-// Sums that the parts cannot vouch for (split_suspect) run the pass again on FP32 MFMAs.
+// Operands are scaled before they are split (split_bf16.hpp); sums that are not finite run the pass
+// again on FP32 MFMAs.
 // SPLIT (small grids, heads from 0): each item's key stages (pass 0's, then pass 1's) are
 // split over two workgroups, neighbours in the XCD order; part 0 writes dQ, part 1 its
 // partial dQ densely into part_ws, and fa2_bwd_dq_sum_kernel adds the two in that order.
@@ -905,7 +927,7 @@ __global__ __launch_bounds__(64 * WAVES, 2) void fa2_bwd_dq_ds_kernel(
       const int f = tid + THREADS * u;
       const int d = f % HS, sh = f / HS;
       bf16x8 p[3];
-      split_bf16(kst[u], p);
+      split_bf16<true>(kst[u], p);
 #pragma unroll
       for (int q = 0; q < 3; ++q)
         *reinterpret_cast<bf16x8*>(
@@ -940,7 +962,7 @@ __global__ __launch_bounds__(64 * WAVES, 2) void fa2_bwd_dq_ds_kernel(
         const float4 lo = dr[sub][2 * st], hi = dr[sub][2 * st + 1];
         const float x[8] = {lo.x, lo.y, lo.z, lo.w, hi.x, hi.y, hi.z, hi.w};
         bf16x8 dp[3];
-        split_bf16(x, dp);
+        split_bf16<true>(x, dp);
 #pragma unroll
         for (int d0 = 0; d0 < HS / 32; d0 += 2) {
           constexpr int ND = HS / 32 < 2 ? 1 : 2;  // two chains
@@ -986,7 +1008,10 @@ __global__ __launch_bounds__(64 * WAVES, 2) void fa2_bwd_dq_ds_kernel(
 
   bool odd = false;
 #pragma unroll
-  for (int d = 0; d < HS / 32; ++d) odd |= split_suspect(acc[d]);
+  for (int d = 0; d < HS / 32; ++d) {
+    odd |= not_finite(acc[d]);
+    acc[d] *= kSplitUnscale * kSplitUnscale;
+  }
   if (__syncthreads_or(odd)) {
     float* const ks = reinterpret_cast<float*>(smem);
 #pragma unroll

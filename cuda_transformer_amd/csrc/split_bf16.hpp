@@ -68,24 +68,4 @@ __device__ __forceinline__ bool not_finite(const f32x16& s) {
 // element, moves an exponent by less than 128 x 2^-134 x 2^85 x log2(e) / sqrt(32) < 2^-42.
 constexpr float kMaxScoreFactor = 0x1p85f;
 
-// Whether a sum of split products may differ from FP32 arithmetic by more than rounding: it is
-// infinite or NaN (an operand was, or rounded to infinity), or nonzero below 2^-100 (operands
-// may have been too small for their low parts).  With u = 2 |bits| and T = 2^-100's, the fine
-// range [T, inf) is one unsigned comparison; exact zeros fail it too and are let off in the
-// second look, which ordinary tiles never reach.
-__device__ __forceinline__ bool split_suspect(const f32x16& s) {
-  constexpr uint32_t T = 27u << 24, kInf = 255u << 24;
-  bool any = false;
-#pragma unroll
-  for (int r = 0; r < 16; ++r) any |= ((__float_as_uint(s[r]) << 1) - T) >= kInf - T;
-  if (!__any(any)) return false;
-  bool bad = false;
-#pragma unroll
-  for (int r = 0; r < 16; ++r) {
-    const uint32_t u = __float_as_uint(s[r]) << 1;
-    bad |= u != 0 && u - T >= kInf - T;
-  }
-  return bad;
-}
-
 }  // namespace cta

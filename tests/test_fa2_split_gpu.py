@@ -136,3 +136,85 @@ def test_forward_small_probabilities_of_large_values(cuda, D):
     ref = _ref(q, k, v, False)
     o, _ = flash_attention_fwd(q.to(cuda), k.to(cuda), v.to(cuda), False)
     assert _rel(o[..., 2], ref[..., 2]) <= 2e-5
+
+
+def _schedules(cuda, q, k, v, dy, causal):
+    """(name, (dq, dk, dv)) through the operator's stored-dS schedule (which splits small grids),
+    the schedule without a workspace and the one that forms delta inside dK/dV."""
+    from cuda_transformer.ops import flash_attention_bwd, flash_attention_fwd
+    from cuda_transformer_amd import capi
+
+    B, H, T, D = q.shape
+    q, k, v, dy = (x.to(cuda) for x in (q, k, v, dy))
+    O, L = flash_attention_fwd(q, k, v, causal)
+    yield "stored", flash_attention_bwd(q, k, v, O, dy, L, causal)
+    s4, s3 = capi.strides(q.stride()), capi.strides(L.stride())
+    st = torch.cuda.current_stream().cuda_stream
+    head = (q.data_ptr(), s4, k.data_ptr(), s4, v.data_ptr(), s4, O.data_ptr(), s4, dy.data_ptr(),
+            s4, L.data_ptr(), s3, B, H, T, D, int(causal))
+    out = [torch.full_like(q, float("nan")) for _ in range(3)]
+    delta = torch.empty(B, H, T, device=cuda)
+    capi.call("cta_flash_attention_bwd", *head, *(t.data_ptr() for t in out), delta.data_ptr(),
+              None, 0, st)
+    yield "recompute", out
+    nbytes = capi.call("cta_flash_attention_bwd_workspace", B, H, T, D, int(causal))
+    ws = torch.empty(nbytes // 4, device=cuda)
+    out = [torch.full_like(q, float("nan")) for _ in range(3)]
+    capi.call("cta_flash_attention_bwd_fold_delta", *head, *(t.data_ptr() for t in out),
+              ws.data_ptr(), nbytes, st)
+    yield "fold_delta", out
+
+
+# Lengths with and without the small-grid split of dK/dV and dQ (T >= 1024; 2048 at hs 32).
+@pytest.mark.parametrize("D,T,causal", [(32, 130, True), (32, 2100, False), (64, 33, False),
+                                        (64, 160, True), (64, 1100, True), (128, 96, True),
+                                        (128, 1100, False)])
+def test_gradients_scaled_operands(cuda, D, T, causal):
+    """Operands whose magnitudes differ by up to 2^240 while the gradients stay in range, rows of
+    dO at 2^-120 among ordinary ones, and gradients that no part can hold: in every schedule."""
+    q, k, v, dy = _qkv(1, 2, T, D, T + D, 4)
+    _, *ref = _ref(q, k, v, causal, dy)
+    for e in (60, 118, -118):
+        for name, (dq, dk, dv) in _schedules(cuda, q * 2.0 ** -e, k * 2.0 ** e, v, dy, causal):
+            got = dq.cpu().double() * 2.0 ** -e, dk.cpu().double() * 2.0 ** e, dv
+            for x, r in zip(got, ref):
+                assert _rel(x, r) <= 1.5e-6, (name, e)
+    for e in (60, 110, -110):
+        for name, (dq, dk, dv) in _schedules(cuda, q, k, v * 2.0 ** e, dy * 2.0 ** -e, causal):
+            for x, r in zip((dq, dk, dv.cpu().double() * 2.0 ** e), ref):
+                assert _rel(x, r) <= 1.5e-6, (name, e)
+    rows = torch.arange(T) % 3 == 1
+    dys = dy.clone()
+    dys[:, :, rows] *= 2.0 ** -120
+    _, *rref = _ref(q, k, v, causal, dys)
+    if causal:
+        rows[0] = False  # its dQ is rounding noise about zero
+    for name, (dq, dk, dv) in _schedules(cuda, q, k, v, dys, causal):
+        for x, r in zip((dq, dk, dv), rref):
+            assert _rel(x, r) <= 1.5e-6, name
+        x, r = dq.cpu().double() * 2.0 ** 120, rref[0] * 2.0 ** 120
+        assert _rel(x[:, :, rows], r[:, :, rows]) <= 3e-6, name
+    for name, got in _schedules(cuda, q, k, v, dy * 2.0 ** -110, causal):
+        for x, r in zip(got, ref):
+            assert _rel(x.cpu().double() * 2.0 ** 110, r) <= 1.5e-6, name
+
+
+@pytest.mark.parametrize("D,T,causal", [(32, 130, True), (32, 2100, False), (64, 160, True),
+                                        (64, 1100, True), (128, 96, True), (128, 1100, False)])
+def test_gradients_second_run_schedules(cuda, D, T, causal):
+    """An infinite entry of dO sends its passes to FP32 MFMAs in every schedule: split dK/dV and dQ,
+    without the dS store, and with delta formed inside."""
+    q, k, v, dy = _qkv(1, 2, T, D, T + D, 4)
+    _, *ref = _ref(q, k, v, causal, dy)
+    i, d = T // 2, 3
+    dy[0, 0, i, d] = float("inf")
+    sees = torch.arange(T) <= (i if causal else T)
+    rows = torch.arange(T) != i
+    for name, got in _schedules(cuda, q, k, v, dy, causal):
+        dq, dk, dv = (x.cpu() for x in got)
+        assert torch.all(dv[0, 0, sees, d] == float("inf")), name
+        dv[0, 0, :, d] = ref[2][0, 0, :, d].float()  # a masked key of the same tile: 0 x inf
+        assert _rel(dv, ref[2]) <= 1.5e-6, name
+        for x, r in ((dq, ref[0]), (dk, ref[1])):
+            assert _rel(x[0, 1], r[0, 1]) <= 1.5e-6, name
+        assert _rel(dq[0, 0, rows], ref[0][0, 0, rows]) <= 1.5e-6, name
