@@ -292,6 +292,15 @@ __global__ __launch_bounds__(256, BwdTile<HS>::MINW) void fa2_bwd_dq_kernel(
 constexpr int kDsTileFloats = 1024;
 constexpr int kDsPitch = 40;  // LDS pitch of the per-wave transpose: halves 4 rows apart hit disjoint banks
 
+// The matrix pipe rounds small addends of a large accumulator downward.  The six products of parts
+// summed over a head of T = 8192 left dQ and dK a mean error of -2.9e-7 of their RMS, which sums
+// over the tokens (bias gradients) show as 18 times what independent roundings leave.  So the
+// stages enter the sum with one sign for kFlipRows rows and the other for the next: the sum is
+// negated in between, and what was rounded down in one run is rounded up in the next (8e-9).  dP's
+// own sums, short but cancelling against delta, take theirs from the block of 32 keys.  (Summing
+// each tile apart and adding it in FP32 has the same effect; its registers cost dK/dV 5-12%.)
+constexpr int kFlipRows = 256;
+
 // ------------------------------------------------------------------------------------
 // Stage 3: dK, dV.  Workgroup = 128 key rows, each of its four waves owning 32 of them and each
 // lane one key row's k and v, as three bfloat16 parts in registers.  All four products run on
@@ -420,21 +429,24 @@ __global__ __launch_bounds__(256, kDkdvMinWaves<HS>) void fa2_bwd_dkdv_kernel(
   const int my_j = j0 + col;
 
   // k's and v's parts, the B operands of S and dP: step st, d 16 st + 8 half + 0..7.
+  // v takes a sign that alternates over the blocks of 32 keys, and with it dP (kFlipRows).
   bf16x8 kp[HS / 16][3], vp[HS / 16][3];
   float kmax = 0.0f;
+  const float v_sign = (j0 >> 5) & 1 ? -1.0f : 1.0f;
 #pragma unroll
   for (int st = 0; st < HS / 16; ++st) {
-    auto load = [&](const float* src, bf16x8 (&p)[3]) {
+    auto load = [&](const float* src, float sign, bf16x8 (&p)[3]) {
       const float4 x = my_j < T ? ld4(src) : zero4(), y = my_j < T ? ld4(src + 4) : zero4();
-      const float v[8] = {x.x, x.y, x.z, x.w, y.x, y.y, y.z, y.w};
+      const float v[8] = {sign * x.x, sign * x.y, sign * x.z, sign * x.w,
+                          sign * y.x, sign * y.y, sign * y.z, sign * y.w};
       split_bf16<true>(v, p);
       float m = 0.0f;
 #pragma unroll
       for (int e = 0; e < 8; e += 2) m = fmaxf(fmaxf(m, fabsf(v[e])), fabsf(v[e + 1]));
       return m;
     };
-    kmax = fmaxf(kmax, load(Kb + (int64_t)my_j * sk.t + 16 * st + 8 * half, kp[st]));
-    load(Vb + (int64_t)my_j * sv.t + 16 * st + 8 * half, vp[st]);
+    kmax = fmaxf(kmax, load(Kb + (int64_t)my_j * sk.t + 16 * st + 8 * half, 1.0f, kp[st]));
+    load(Vb + (int64_t)my_j * sv.t + 16 * st + 8 * half, v_sign, vp[st]);
   }
   // The pass runs again on FP32 MFMAs.  (The vote is taken here: left to the end of the pass, it
   // would keep k in registers.)
@@ -598,9 +610,16 @@ __global__ __launch_bounds__(256, kDkdvMinWaves<HS>) void fa2_bwd_dkdv_kernel(
   const bool down = CAUSAL && kt <= n_ktiles - 1 - kt;
   auto stage_at = [&](int i) { return down ? n_stages - 1 - i : q_begin + i; };
   if (i_begin < i_end) issue(stage_at(i_begin), rvec[slot]);
-  constexpr float y = kSplitScale;  // the scale of P and dS in the sums
+  constexpr int kFlip = kFlipRows / BN;
+  float y = kSplitScale;  // the scale, and now and then the sign, of P and dS in the sums
 
-  for (int i = i_begin; i < i_end; ++i) {
+  for (int run = i_begin; run < i_end; run += kFlip) {
+  if (run > i_begin) {
+    y = -y;
+#pragma unroll
+    for (int d = 0; d < HS / 32; ++d) { dkacc[d] = -dkacc[d]; dvacc[d] = -dvacc[d]; }
+  }
+  for (int i = run; i < min(run + kFlip, i_end); ++i) {
     // the stage's copies have landed, and every wave is done with the images
     vm_wait_all();
     __syncthreads();
@@ -662,16 +681,18 @@ __global__ __launch_bounds__(256, kDkdvMinWaves<HS>) void fa2_bwd_dkdv_kernel(
     };
     probabilities(sacc, ii0, rv, scale_log2 * kSplitUnscale, y);
     accumulate(dvacc, images + 3 * IMAGE, sacc);
-    score_gradients(sacc, pacc, rv + RVEC, kSplitUnscale * kSplitUnscale);
+    score_gradients(sacc, pacc, rv + RVEC, v_sign * (kSplitUnscale * kSplitUnscale));
     if (STORE_DS) store_ds(pacc, ii0, y * (kSplitUnscale * kSplitUnscale));
     accumulate(dkacc, images + 2 * IMAGE, pacc);
   }
+  }  // run
 
+  y *= kSplitUnscale * kSplitUnscale * kSplitUnscale;
 #pragma unroll
   for (int d = 0; d < HS / 32; ++d) {
     odd |= not_finite(dkacc[d]) || not_finite(dvacc[d]);
-    dkacc[d] *= kSplitUnscale * kSplitUnscale;
-    dvacc[d] *= kSplitUnscale * kSplitUnscale;
+    dkacc[d] *= y;
+    dvacc[d] *= y;
   }
   vm_wait_all();  // dS tiles that a second run stores again are stored in order
   if (__syncthreads_or(odd)) {
@@ -952,6 +973,8 @@ __global__ __launch_bounds__(64 * WAVES, 2) void fa2_bwd_dq_ds_kernel(
       }
     }
   };
+  constexpr int kFlip = kFlipRows / BN;  // even
+  float y = kSplitScale;  // the scale, and now and then the sign, of dS in the sums
   auto compute = [&](int stage, const char* ks, const float4 (&dr)[NSUB][4]) {
     if (stage >= s_end) return;  // a padded stage (or, split, the other part's)
 #pragma unroll
@@ -960,9 +983,10 @@ __global__ __launch_bounds__(64 * WAVES, 2) void fa2_bwd_dq_ds_kernel(
 #pragma unroll
       for (int st = 0; st < 2; ++st) {
         const float4 lo = dr[sub][2 * st], hi = dr[sub][2 * st + 1];
-        const float x[8] = {lo.x, lo.y, lo.z, lo.w, hi.x, hi.y, hi.z, hi.w};
+        const float x[8] = {y * lo.x, y * lo.y, y * lo.z, y * lo.w,
+                            y * hi.x, y * hi.y, y * hi.z, y * hi.w};
         bf16x8 dp[3];
-        split_bf16<true>(x, dp);
+        split_bf16(x, dp);
 #pragma unroll
         for (int d0 = 0; d0 < HS / 32; d0 += 2) {
           constexpr int ND = HS / 32 < 2 ? 1 : 2;  // two chains
@@ -999,18 +1023,26 @@ __global__ __launch_bounds__(64 * WAVES, 2) void fa2_bwd_dq_ds_kernel(
     lstore(0);
     __syncthreads();
     // Unrolled by two so the two dS register sets swap roles without copies.
-    const int n_run2 = (s_end - s_begin + 1) & ~1;
-    for (int s = s_begin; s < s_begin + n_run2; s += 2) {
-      step(s, dA, dB);
-      step(s + 1, dB, dA);
+    const int s_end2 = s_begin + ((s_end - s_begin + 1) & ~1);
+    for (int run = s_begin; run < s_end2; run += kFlip) {
+      if (run > s_begin) {
+        y = -y;
+#pragma unroll
+        for (int d = 0; d < HS / 32; ++d) acc[d] = -acc[d];
+      }
+      for (int s = run; s < min(run + kFlip, s_end2); s += 2) {
+        step(s, dA, dB);
+        step(s + 1, dB, dA);
+      }
     }
   }
 
   bool odd = false;
+  y *= kSplitUnscale * kSplitUnscale * kSplitUnscale;
 #pragma unroll
   for (int d = 0; d < HS / 32; ++d) {
     odd |= not_finite(acc[d]);
-    acc[d] *= kSplitUnscale * kSplitUnscale;
+    acc[d] *= y;
   }
   if (__syncthreads_or(odd)) {
     float* const ks = reinterpret_cast<float*>(smem);

@@ -218,3 +218,23 @@ def test_gradients_second_run_schedules(cuda, D, T, causal):
         for x, r in ((dq, ref[0]), (dk, ref[1])):
             assert _rel(x[0, 1], r[0, 1]) <= 1.5e-6, name
         assert _rel(dq[0, 0, rows], ref[0][0, 0, rows]) <= 1.5e-6, name
+
+
+@pytest.mark.parametrize("D,T,H,causal", [(64, 4096, 4, False), (64, 4096, 64, True), (32, 4096, 4, True),
+                                          (128, 2048, 4, False)])
+def test_gradient_column_sums(cuda, D, T, H, causal):
+    """Rounding of dQ and dK has no sign of its own: the sums over the tokens (a bias gradient) are
+    off by no more than independent errors of the gradients' own size would leave, three of their
+    standard deviations.  A matrix pipe that rounds small addends of a large accumulator downward
+    left nine at T = 4096."""
+    from cuda_transformer.ops import flash_attention_bwd, flash_attention_fwd
+
+    q, k, v, dy = _qkv(1, H, T, D, T + D, 4)
+    dev = [x.to(cuda) for x in (q, k, v, dy)]
+    O, L = flash_attention_fwd(*dev[:3], causal)
+    got = flash_attention_bwd(*dev[:3], O, dev[3], L, causal)
+    _, *ref = _ref(*(x[:, :2] for x in (q, k, v)), causal, dy[:, :2])
+    for name, x, r in zip("qk", got, ref):
+        e = x[:, :2].double().cpu() - r
+        drift = float(e.sum(2).norm() / (r.norm()))  # sqrt(T) sigma, over sqrt(T) rms
+        assert drift <= 3 * float(e.norm() / r.norm()), (name, drift)
