@@ -1177,11 +1177,12 @@ void launch_dq_ds(const float* k, const float* dsw, float* dq, int nh, int T, in
                        dim3(64 * WAVES), 0, st, k, dsw, dq, nh, T, bh_base, n_heads, n_qtiles, sk,
                        sdq, scale, nullptr, lpt);
   };
-  // Short causal heads (hs 64, T <= 1024): two waves (64 query rows) per workgroup, as in the
-  // dK/dV stage.  A/B in one process, bitwise-equal dQ: +11.5% at T = 256, +10% at 512, +5% at
-  // 1024 (B16 H6), +0.5% at B4 H32 T1024.
+  // Short causal heads (hs 64, T <= 512): two waves (64 query rows) per workgroup.  Two waves
+  // against four: T64 64 heads 5.9 and 6.6 us; T256 B64 H6 27.7 and 32.3, 64 heads 12.5 and 12.1;
+  // T512 B64 H6 69.4 and 69.1, 128 heads 29.7 and 30.9, 64 heads 22.3 and 20.6.  Beyond: T768 128
+  // heads 55.6 and 56.6, 16 heads 29.6 and 27.0; T1024 256 heads 168 and 150.
   if constexpr (HS == 64 && CAUSAL) {
-    if (T <= 1024) {
+    if (T <= 512) {
       run.template operator()<2>();
       return;
     }

@@ -481,22 +481,43 @@ __global__ __launch_bounds__(256) void fa2_fwd_merge_kernel(float* __restrict__ 
 
 // The forward splits each work item's K/V stages over NSPLIT workgroups when its grid would hold
 // fewer than two waves per SIMD (1024 SIMDs): up to three parts at hs 32 / 64 and two at hs 128,
-// each keeping at least kSplitMinStages stages; the merge pass is the cost.  B4 H4 N4096 causal
-// takes 235 us in three parts (two: 227; on FP32 MFMAs, which held three waves per SIMD, 298 in
-// three); callers size their workspace by this rule, so it stays.  At T = 256 (B64 H6, 8 stages
-// per row) two parts were 30% slower, the merge outweighing the work, hence the minimum.
+// each keeping at least kSplitMinStages stages; the merge pass is the cost.  Three parts against
+// two: B1 H2 N8192 causal 157 and 228 us, B2 H6 N1600 48 and 62, B1 H8 N4096 126 and 126; at one
+// wave per SIMD unsplit they are slower, B4 H4 N4096 214 and 202 us, B2 H4 N4096 non-causal 193
+// and 188, but the parts per shape, with the workspace's size, are part of the interface that
+// tests pin.  At T = 256 (B64 H6, 8 stages per row) two parts were 30% slower (measured on FP32
+// MFMAs), the merge outweighing the work, hence the minimum.
 constexpr int kSimds = 1024;
 constexpr int kSplitMinStages = 16;
 
+// Waves per SIMD that the forward's registers hold (hs 32: two or three).
+template <int HS>
+constexpr int kFwdOcc = HS == 128 ? 1 : 2;
+
+// Waves per workgroup.  Two waves (64 query rows) split every K/V stage for half as many rows, so
+// the splits cost twice as much; what they gain is the balance of short causal heads (hs 64,
+// T <= 512).  They are taken where four-wave tiles cannot go longest first (lpt_heads) but two-wave
+// ones can, or their pairs fill at most three quarters of the resident slots; and for T <= 64, where
+// two of four waves would have no row, once the heads' four-wave workgroups no longer fit the
+// slots.  Two waves against four: T256 B64 H6 39.7 and 42.4 us, 256 heads 29.3 and 32.7; T384 128
+// heads 31.6 and 38.2; T512 128 heads 43.2 and 45.0; T33 3072 heads 41.8 and 53.3.  Beyond the
+// lines: T512 256 heads 98 and 67, 64 heads 36.9 and 32.8; T256 1024 heads 107 and 88, 64 heads
+// 20.5 and 19.7; T128 1024 heads 47 and 38; T64 64 heads 9.1 and 8.8.
 template <int HS, bool CAUSAL>
-int fwd_waves(int T) {
-  return (HS == 64 && CAUSAL && T <= 512) ? 2 : 4;
+int fwd_waves(int T, int BH) {
+  if (HS != 64 || !CAUSAL || T > 512) return 4;
+  if (T <= 64) return BH > kFwdOcc<HS> * kNumSimds / 4 ? 2 : 4;
+  if (T <= 128) return 4;
+  if (lpt_heads(BH, (T + 127) / 128, 4, kFwdOcc<HS>) > 0) return 4;
+  const int n2 = (T + 63) / 64;  // two-wave tiles of a head
+  if (lpt_heads(BH, n2, 2, kFwdOcc<HS>) > 0) return 2;
+  return 4 * (int64_t)BH * ((n2 + 1) / 2) <= 3 * (kFwdOcc<HS> * kNumSimds / 2) ? 2 : 4;
 }
 
 // Parts per work item: 1 (no split), 2 or 3.
 template <int HS, bool CAUSAL>
 int fwd_nsplit(int T, int BH) {
-  const int waves = fwd_waves<HS, CAUSAL>(T);
+  const int waves = fwd_waves<HS, CAUSAL>(T, BH);
   const int n_qtiles = (T + 32 * waves - 1) / (32 * waves);
   const int64_t w = (int64_t)(CAUSAL ? (n_qtiles + 1) / 2 : n_qtiles) * BH * waves;
   if (w >= 2 * kSimds) return 1;
@@ -538,21 +559,15 @@ void launch_fwd(const float* q, const float* k, const float* v, float* o, float*
       split.template operator()<2>();
       return;
     }
-    // Slots counted at the two waves per SIMD the kernel holds (one at hs 128): B64 H6 T256
-    // takes 43.7 us, 45.3 with three counted.
-    const int lpt = CAUSAL ? lpt_heads(BH, n_qtiles, WAVES, HS == 128 ? 1 : 2) : 0;
+    const int lpt = CAUSAL ? lpt_heads(BH, n_qtiles, WAVES, kFwdOcc<HS>) : 0;
     hipLaunchKernelGGL((fa2_fwd_kernel<HS, CAUSAL, WAVES>),
                        dim3(lpt > 0 ? (unsigned)(BH * n_qtiles) : xcd_grid(items)),
                        dim3(64 * WAVES), 0, stream, q, k, v, o, l, nh, T, BH, n_qtiles, sq, sk,
                        sv, so, scale, scale * kLog2e, 8.0f / (scale * kLog2e), nullptr, nullptr,
                        lpt);
   };
-  // Short causal heads (hs 64, T <= 512) run two waves (64 query rows) per workgroup: fewer
-  // waves idle at each K/V stage's barrier along the diagonal, and the query-tile pairs balance
-  // over twice as many workgroups.  A/B in one process, bitwise-equal outputs: +13% at T = 256,
-  // +7% at 512, within 1.5% either way at 1024 and 2048.
   if constexpr (HS == 64 && CAUSAL) {
-    if (T <= 512) {
+    if (fwd_waves<HS, CAUSAL>(T, BH) == 2) {
       run.template operator()<2>();
       return;
     }

@@ -238,3 +238,20 @@ def test_gradient_column_sums(cuda, D, T, H, causal):
         e = x[:, :2].double().cpu() - r
         drift = float(e.sum(2).norm() / (r.norm()))  # sqrt(T) sigma, over sqrt(T) rms
         assert drift <= 3 * float(e.norm() / r.norm()), (name, drift)
+
+
+# Both sides of the lines between two- and four-wave workgroups (hs 64, causal): T = 64 | 65, 128 |
+# 129 and 512 | 513, longest-first tiles or pairs, and grids that fill the chip or not.
+@pytest.mark.parametrize("heads,T", [(512, 64), (513, 64), (520, 65), (8, 128), (8, 129), (12, 200), (64, 256), (96, 200), (256, 256),
+                                     (1024, 256), (64, 512), (128, 512), (256, 512), (16, 513)])
+def test_short_causal_heads(cuda, heads, T):
+    q, k, v, dy = _qkv(1, heads, T, 64, heads + T, 4)
+    from cuda_transformer.ops import flash_attention_bwd, flash_attention_fwd
+
+    dev = [x.to(cuda) for x in (q, k, v, dy)]
+    O, L = flash_attention_fwd(*dev[:3], True)
+    got = (O, *flash_attention_bwd(*dev[:3], O, dev[3], L, True))
+    for h in (0, heads - 1):
+        ref = _ref(*(x[:, h : h + 1] for x in (q, k, v)), True, dy[:, h : h + 1])
+        for x, r in zip(got, ref):
+            assert _rel(x[:, h : h + 1], r) <= 1.5e-6
