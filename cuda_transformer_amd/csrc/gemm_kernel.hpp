@@ -410,7 +410,7 @@ __device__ __forceinline__ void block_store(const f32x16 (&acc)[TL::MB][TL::NB],
 template <class TL, class PA, class PB>
 __device__ __forceinline__ void exact_tile(const PA& pa, const PB& pb, typename PA::S& la,
                                            typename PB::S& lb, float* smem, int nk, int tid,
-                                           int wm, int wn, int half, int col,
+                                           int tid_b, int wm, int wn, int half, int col,
                                            f32x16 (&acc)[TL::MB][TL::NB]) {
   constexpr int BM = TL::BM, BN = TL::BN;
 #pragma unroll
@@ -419,11 +419,11 @@ __device__ __forceinline__ void exact_tile(const PA& pa, const PB& pb, typename 
     for (int j = 0; j < TL::NB; ++j) acc[i][j] = zero16();
   float* const as = smem;
   float* const bs = smem + kGemmK * BM;
-  auto put = [&](const auto& plan, const auto& L, float* lds, int rows) {
+  auto put = [&](const auto& plan, const auto& L, float* lds, int rows, int id) {
     using S = std::remove_cvref_t<decltype(L)>;
 #pragma unroll
     for (int u = 0; u < S::N; ++u) {
-      const int f = tid + TL::THREADS * u;
+      const int f = id + TL::THREADS * u;
       if (f >= S::UNITS) continue;
       int r, h;
       plan.coords(f, r, h);
@@ -433,12 +433,12 @@ __device__ __forceinline__ void exact_tile(const PA& pa, const PB& pb, typename 
   };
   for (int t = 0; t < nk; ++t) {
     pa.load(la, t, tid);
-    pb.load(lb, t, tid);
+    pb.load(lb, t, tid_b);
     pa.mask(la, t);
     pb.mask(lb, t);
     __syncthreads();
-    put(pa, la, as, BM);
-    put(pb, lb, bs, BN);
+    put(pa, la, as, BM, tid);
+    put(pb, lb, bs, BN, tid_b);
     __syncthreads();
 #pragma unroll
     for (int e = 0; e < kGemmK / 2; ++e) {
@@ -473,6 +473,8 @@ __global__ __launch_bounds__(TL::THREADS, 2) void gemm_kernel(GemmOperand A, Gem
   constexpr int MB = TL::MB, NB = TL::NB;
   __shared__ __attribute__((aligned(16))) char smem[2 * TL::BUF_BYTES];
   const int tid = threadIdx.x;
+  // Where half of the threads hold an operand's slice (the 64x64 tile), the other half holds B's.
+  const int tid_b = 2 * BM + 2 * BN <= THREADS ? tid ^ (2 * BM) : tid;
   const int lane = tid & 63, wave = wave_index();
   const int half = lane >> 5, col = lane & 31;
   const int wm = wave / TL::WN, wn = wave % TL::WN;
@@ -513,7 +515,7 @@ __global__ __launch_bounds__(TL::THREADS, 2) void gemm_kernel(GemmOperand A, Gem
   PlanA pa;
   PlanB pb;
   pa.init(Ab, A.s_row, A.s_col, m0, kb, M, ke, tid);
-  pb.init(Bb, B.s_col, B.s_row, n0, kb, N, ke, tid);
+  pb.init(Bb, B.s_col, B.s_row, n0, kb, N, ke, tid_b);
   typename PlanA::S la0, la1;
   typename PlanB::S lb0, lb1;
   const int nk = (ke - kb + kGemmK - 1) / kGemmK;
@@ -550,13 +552,13 @@ __global__ __launch_bounds__(TL::THREADS, 2) void gemm_kernel(GemmOperand A, Gem
   char* const buf0 = smem;
   char* const buf1 = smem + TL::BUF_BYTES;
   pa.load(la0, 0, tid);
-  pb.load(lb0, 0, tid);
+  pb.load(lb0, 0, tid_b);
   pa.load(la1, 1, tid);
-  pb.load(lb1, 1, tid);
+  pb.load(lb1, 1, tid_b);
   pa.mask(la0, 0);
   pb.mask(lb0, 0);
   store_slice<AMODE, BM, THREADS, PA>(la0, buf0, tid);
-  store_slice<BMODE, BN, THREADS, PB>(lb0, buf0 + TL::A_BYTES, tid);
+  store_slice<BMODE, BN, THREADS, PB>(lb0, buf0 + TL::A_BYTES, tid_b);
   add_cs(lb0);
   __syncthreads();
 
@@ -572,12 +574,12 @@ __global__ __launch_bounds__(TL::THREADS, 2) void gemm_kernel(GemmOperand A, Gem
                    typename PlanB::S& lb_far, typename PlanA::S& la_next,
                    typename PlanB::S& lb_next, char* nbuf, int t_far) {
     pa.load(la_far, t_far, tid);
-    pb.load(lb_far, t_far, tid);
+    pb.load(lb_far, t_far, tid_b);
     mma_products<TL, 0, 3>(cur, acc, low);
     pa.mask(la_next, t_far - 1);
     pb.mask(lb_next, t_far - 1);
     store_slice<AMODE, BM, THREADS, PA>(la_next, nbuf, tid);
-    store_slice<BMODE, BN, THREADS, PB>(lb_next, nbuf + TL::A_BYTES, tid);
+    store_slice<BMODE, BN, THREADS, PB>(lb_next, nbuf + TL::A_BYTES, tid_b);
     add_cs(lb_next);
     __syncthreads();
     read_frags<TL>(nbuf, nxt, wm, wn, half, col);
@@ -600,8 +602,8 @@ __global__ __launch_bounds__(TL::THREADS, 2) void gemm_kernel(GemmOperand A, Gem
       acc[i][j] *= kSplitUnscale * kSplitUnscale;
     }
   if (__syncthreads_or(odd))
-    exact_tile<TL>(pa, pb, la0, lb0, reinterpret_cast<float*>(smem), nk, tid, wm, wn, half, col,
-                   acc);
+    exact_tile<TL>(pa, pb, la0, lb0, reinterpret_cast<float*>(smem), nk, tid, tid_b, wm, wn, half,
+                   col, acc);
 
   if constexpr (CS) {
     if (m0 == 0) {  // workgroup-uniform
@@ -614,7 +616,7 @@ __global__ __launch_bounds__(TL::THREADS, 2) void gemm_kernel(GemmOperand A, Gem
       __syncthreads();  // every wave is done with the slices
 #pragma unroll
       for (int u = 0; u < PlanB::N; ++u) {
-        const int f = tid + THREADS * u;
+        const int f = tid_b + THREADS * u;
         if (f >= BN && f < 2 * BN) half1[f - BN] = unit_sum(u);
       }
       __syncthreads();
@@ -622,7 +624,7 @@ __global__ __launch_bounds__(TL::THREADS, 2) void gemm_kernel(GemmOperand A, Gem
                             : ep.colsum;
 #pragma unroll
       for (int u = 0; u < PlanB::N; ++u) {
-        const int f = tid + THREADS * u;
+        const int f = tid_b + THREADS * u;
         if (f < BN && n0 + f < N) out[n0 + f] = unit_sum(u) + half1[f];
       }
     }
