@@ -18,14 +18,22 @@ int gemm_launch(const GemmOperand& A, const GemmOperand& B, const GemmOut& C,
   if (S > 1 && workspace != nullptr &&
       workspace_floats >= S * (Z * M * N + (ep.colsum ? N : 0)))
     return gemm_launch_wide(A, B, C, ep, M, N, K, Z, zin, st, workspace, workspace_floats);
-  // Small outputs: 64x64 tiles while 64x128 ones would leave CUs without a workgroup (195 x 1155
-  // x 385: 20 us against 27 with 128x128 tiles).  Otherwise 64x128 for narrow outputs (16384 x
-  // 384 x 1536: 126 us, 132 with 128x128; 8192 x 768 x 3072: 248 against 262) and 128x128 for
-  // wide ones (8192 x 3072 x 768: 209 us, 239 with 64x128).  The tile never depends on the
-  // pointwise stage, and all of them sum in the same order.
-  const int64_t narrow_tiles = (M + 63) / 64 * ((N + 127) / 128) * Z;
-  if (narrow_tiles < 256) return gemm_launch_small(A, B, C, ep, M, N, K, Z, zin, st, nullptr, 0);
-  if (N <= 768) return gemm_launch_narrow(A, B, C, ep, M, N, K, Z, zin, st, nullptr, 0);
+  // The tile goes by how many there are: 256 CUs hold one, two or three workgroups of each at once.
+  // 64x64 up to 640 tiles (2048 x 1152 x 384, W transposed: 20.6 us, 64x128 23.4, 128x128 22.0) and
+  // while 64x128 ones would leave CUs without a workgroup (195 x 1155 x 385: 16, 21 and 25).
+  // 64x128 where 128x128 would leave most CUs one workgroup and some two (2048 x 2304 x 384: 31.8
+  // us, 128x128 34.2; 8192 x 576 x 384 32.8 and 34.5) and the loads are the ones whose kernels hold
+  // three workgroups a CU (the weight gradient's 64x128 kernel holds two: 1216 x 3456 x 14775 1571
+  // us, 128x128 1030).  Otherwise 128x128 (16384 x 768 x 384: 60 us, 64x128 68; 8192 x 1536 x 384 61 and 68;
+  // 8192 x 384 x 384 23.9 and 25.2).  The tile never depends on the pointwise stage, and all of them
+  // sum in the same order.
+  const int64_t m64 = (M + 63) / 64 * Z, n128 = (N + 127) / 128;
+  const int64_t wide = (M + 127) / 128 * Z * n128;
+  if (m64 * n128 < 256 || m64 * ((N + 63) / 64) <= 640)
+    return gemm_launch_small(A, B, C, ep, M, N, K, Z, zin, st, nullptr, 0);
+  if (wide > 256 && wide <= 320 && pick_mode(A, true, M, K) == kVecK &&
+      pick_mode(B, false, N, K) <= kVecMN)
+    return gemm_launch_narrow(A, B, C, ep, M, N, K, Z, zin, st, nullptr, 0);
   return gemm_launch_wide(A, B, C, ep, M, N, K, Z, zin, st, nullptr, 0);
 }
 

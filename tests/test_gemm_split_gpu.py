@@ -155,3 +155,16 @@ def test_weight_bias_grad_column_strides(cuda):
     dw, db = (t.double().cpu() for t in linear_weight_bias_grad(x.to(cuda), wide.to(cuda)[..., 0]))
     assert torch.all((dw - x.double().t() @ dy.double()).abs() <= _bound(x.t(), dy))
     assert torch.all((db - dy.double().sum(0)).abs() <= 1e-6 * dy.double().abs().sum(0))
+
+
+# Both sides of the tile choice's lines: 640 | 672 tiles of 64x64, 256 | 288, 320 | 352 tiles of
+# 128x128, and the operand orders that never take 64x128.
+@pytest.mark.parametrize("order", ["nn", "nt", "tn"])
+@pytest.mark.parametrize("m,k,n", [(2048, 48, 1280), (2048, 48, 1344), (4096, 48, 1024), (4096, 52, 1152),
+                                   (4096, 48, 1280), (4096, 52, 1408), (4096, 35, 1152)])
+def test_gemm_tile_lines(cuda, m, k, n, order):
+    from cuda_transformer.ops import cuda_fma
+
+    x, w, xc, wc = _operands(m, k, n, order, m + k + n)
+    out = cuda_fma(xc, wc, torch.zeros(n, device=cuda))[0].double().cpu()
+    assert torch.all((out - x.double() @ w.double()).abs() <= _bound(x, w))
