@@ -581,6 +581,19 @@ __global__ __launch_bounds__(TL::THREADS, 2) void gemm_kernel(GemmOperand A, Gem
     store_slice<AMODE, BM, THREADS, PA>(la_next, nbuf, tid);
     store_slice<BMODE, BN, THREADS, PB>(lb_next, nbuf + TL::A_BYTES, tid_b);
     add_cs(lb_next);
+    if constexpr (PlanA::S::UNITS % THREADS == 0 && PlanB::S::UNITS % THREADS == 0) {
+      // Each MFMA takes the pipe for eight vector instructions' time: the slice's splits go
+      // between them, evenly.  Left alone, the scheduler ran most of every second slice's after
+      // the last MFMA (4096 x 3072 x 1536: 214 us, 198 so; one workgroup a CU, 2048 x 2048 x 2048:
+      // 107 and 98).
+      constexpr int kMfmas = 6 * MB * NB;
+      constexpr int kValu = 52 * (PlanA::N + PlanB::N);
+#pragma unroll
+      for (int i = 0; i < kMfmas; ++i) {
+        __builtin_amdgcn_sched_group_barrier(0x008, 1, 0);  // MFMA
+        __builtin_amdgcn_sched_group_barrier(0x002, (kValu + kMfmas - 1) / kMfmas, 0);  // VALU
+      }
+    }
     __syncthreads();
     read_frags<TL>(nbuf, nxt, wm, wn, half, col);
     mma_products<TL, 3, 6>(cur, acc, low);
