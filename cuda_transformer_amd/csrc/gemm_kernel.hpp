@@ -581,11 +581,14 @@ __global__ __launch_bounds__(TL::THREADS, 2) void gemm_kernel(GemmOperand A, Gem
     store_slice<AMODE, BM, THREADS, PA>(la_next, nbuf, tid);
     store_slice<BMODE, BN, THREADS, PB>(lb_next, nbuf + TL::A_BYTES, tid_b);
     add_cs(lb_next);
-    if constexpr (PlanA::S::UNITS % THREADS == 0 && PlanB::S::UNITS % THREADS == 0) {
+    if constexpr (PlanA::S::UNITS % THREADS == 0 && PlanB::S::UNITS % THREADS == 0 &&
+                  !(AMODE == kStrided && BMODE == kVecK)) {
       // Each MFMA takes the pipe for eight vector instructions' time: the slice's splits go
       // between them, evenly.  Left alone, the scheduler ran most of every second slice's after
       // the last MFMA (4096 x 3072 x 1536: 214 us, 198 so; one workgroup a CU, 2048 x 2048 x 2048:
-      // 107 and 98).
+      // 107 and 98).  Strided A beside W^T's rows is left to the scheduler: its eight single loads a
+      // unit, issued between the MFMAs too, and full registers wait (2048 x 768 x 3072: 116 us
+      // interleaved, 106 not).
       constexpr int kMfmas = 6 * MB * NB;
       constexpr int kValu = 52 * (PlanA::N + PlanB::N);
 #pragma unroll
