@@ -1,8 +1,9 @@
 // Shared device helpers and host-side error plumbing for the gfx950 kernels.
 //
-// Every kernel in this library is written for CDNA4 (gfx950): wave64, FP32 MFMA
-// (v_mfma_f32_32x32x2_f32), LDS tiles with padded pitches.  The lane layout of the
-// 32x32x2 MFMA that all attention / GEMM kernels rely on (checked on an MI355X):
+// Every kernel in this library is written for CDNA4 (gfx950): wave64, MFMA, LDS tiles.  FP32
+// products mostly run on the BF16 MFMA (split_bf16.hpp); dQ of the recompute schedule and second
+// runs use the FP32 one.  The lane layout of the 32x32x2 FP32 MFMA (checked on an MI355X; the
+// 16-bit 32x32x16 MFMAs have the same output layout):
 //   A operand (32 x 2):  lane l supplies A[l % 32][l / 32]
 //   B operand (2 x 32):  lane l supplies B[l / 32][l % 32]
 //   D (32 x 32, 16 regs): lane l, register r holds D[R(r, l/32)][l % 32]
@@ -192,9 +193,9 @@ __device__ __forceinline__ void lpt_tile(int hw_id, int heads_per_xcd, int& bh, 
 // the pairs: longest-first tiles there measured 1-2% faster in short bursts, but the tiles that
 // the dispatcher starts one by one no longer share K/V stages (L2 misses 3-4x: forward 0.65 ->
 // 2.9 GB at B4 H32 N4096), and under sustained load, which holds the chip at its power limit,
-// the gain was gone.  With several four-wave tiles on one CU the unequal tiles that share it
-// cost more than a pair.  `waves` per workgroup, `occ` waves per SIMD the kernel holds; BH must
-// split evenly over the XCDs.
+// the gain was gone (the FP32 kernels when their products ran on FP32 MFMAs, and the 16-bit ones).
+// With several four-wave tiles on one CU the unequal tiles that share it cost more than a pair.
+// `waves` per workgroup, `occ` waves per SIMD the kernel holds; BH must split evenly over the XCDs.
 constexpr int kNumSimds = 1024;
 inline int lpt_heads(int64_t BH, int n_tiles, int waves, int occ) {
   if (BH % kNumXcds != 0 || n_tiles < 2) return 0;

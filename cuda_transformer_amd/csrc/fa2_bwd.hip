@@ -312,7 +312,8 @@ constexpr int kFlipRows = 256;
 // into four images in MFMA operand order, Q and dO by rows (S, dP) and by columns (dK, dV).  One
 // image set (48 KiB at hs 64) and one FP32 stage leave room for two workgroups a CU, which hide
 // each other's two barriers a stage; a second image set would leave one.
-// B4 H32 N4096 D64 causal: 4.2 -> 3.2 ms, MFMA busy 55% at 1.86 GHz; B2 H16 T1999 D128 0.52 ms.
+// B4 H32 N4096 D64 causal: 4.2 -> 3.2 ms with the dS store (2.7 without), MFMA busy 53% at
+// 1.84 GHz; B2 H16 T1999 D128 0.44 ms.  (hs 64 spills 44-60 bytes outside the stage loop.)
 // The rest is VALU work (the splits and the softmax, about 600 instructions a tile, in long runs
 // between the MFMAs), the barriers and the chip's power limit.
 //
@@ -335,7 +336,7 @@ constexpr int kFlipRows = 256;
 // finite (infinities, NaN, operands above 2^103, dK or dV above 2^79, dP above 2^79), or |k| above
 // kMaxScoreFactor, run the pass again on FP32 MFMAs: a P or dS that is not finite leaves its key's
 // dV or dK not finite, so these two are all that is looked at.  With every pass run again the
-// backward takes 2.4 to 2.6 times as long.
+// backward takes 2.3 to 2.6 times as long.
 template <int HS, bool CAUSAL, bool STORE_DS, bool FOLD, bool SPLIT = false>
 __global__ __launch_bounds__(256, kDkdvMinWaves<HS>) void fa2_bwd_dkdv_kernel(
     const float* __restrict__ Q, const float* __restrict__ K, const float* __restrict__ V,
@@ -825,8 +826,9 @@ __global__ __launch_bounds__(256) void fa2_bwd_dq_sum_kernel(float* __restrict__
 // matrix pipe, six products of three-part operands (split_bf16.hpp; 768 matrix cycles a tile at
 // hs 64, 2048 on the FP32 MFMA).  K stages go global -> registers -> split -> LDS, double
 // buffered; each wave streams its own dS tiles from the workspace straight into registers,
-// one stage ahead, and splits them there as the B operand.  What bounds it is the read of dS: B1 H32 N8192 D64
-// 2.29 -> 1.58 ms (5.6 TB/s), B4 H32 N4096 causal 1.26 -> 0.91 ms.
+// one stage ahead, and splits them there as the B operand.  What bounds it is mostly the read of
+// dS, at the chip's power limit: B1 H32 N8192 D64 2.29 -> 1.67-1.89 ms (4.5-5.3 TB/s, MFMA busy 52%),
+// B4 H32 N4096 causal 1.26 -> 0.92-0.98 ms.
 // A stage is 64 keys, or 32 where two buffers of 64 would hold the CU to fewer than three
 // workgroups of four waves (hs 128; two-wave workgroups).  Heads [bh_base, bh_base + BH).
 // Operands are scaled before they are split (split_bf16.hpp); sums that are not finite run the pass

@@ -9,8 +9,8 @@
 //    causal heads).  Both products run on the BF16 matrix pipe with FP32 operands split into
 //    three bfloat16 parts, six products of parts each (gemm_kernel.hpp): 1536 matrix cycles per
 //    32x32 score tile at hs 64 where the FP32 MFMA takes 4096.  At B4 H32 N4096 D64 causal the
-//    forward takes 1.51 ms (182 TFLOP/s), 2.18 on FP32 MFMAs, with an error against float64 of
-//    2.1e-7 instead of 5.0e-7.  What bounds it: the VALU work beside the MFMAs (the softmax and
+//    forward takes 1.43 ms (192 TFLOP/s), 2.18 on FP32 MFMAs, with an error against float64 of
+//    2.0e-7 instead of 5.0e-7.  What bounds it: the VALU work beside the MFMAs (the softmax and
 //    the splits of P, K and V, about 900 of each tile's cycles) at two waves per SIMD, and the
 //    chip's power limit.
 //  * K/V stages of 32 rows go global -> registers -> split -> LDS, double buffered, one barrier
@@ -24,9 +24,9 @@
 //    that order.  P never leaves registers.
 //  * Q, P and V are scaled by 2^24 before they are split, so their parts hold every bit of them
 //    (split_bf16.hpp); K's may lack what lies below 2^-133, which moves no score that matters
-//    while |q| < 2^85 (kMaxScoreFactor).  A pass with a larger q, or whose sums are not finite, is run again on
-//    FP32 MFMAs by the whole workgroup, so infinities, NaN and values up to FP32's largest give
-//    what FP32 arithmetic gives.
+//    while |q| < 2^85 (kMaxScoreFactor).  A pass with a larger q, or whose sums are not finite, is
+//    run again on FP32 MFMAs by the whole workgroup (2.6-3.0 times the time), so infinities, NaN
+//    and values up to FP32's largest give what FP32 arithmetic gives.
 //  * Exponentials use exp2 with log2(e) folded into the scale; L is exported in natural log.
 //  * Lazy rescaling: the running max m used as the exponent offset only moves when some row
 //    of the wave sees a tile max more than 2^8 above it (a wave-uniform vote).  Otherwise the
@@ -527,10 +527,9 @@ int fwd_nsplit(int T, int BH) {
   return n >= 2 ? n : 1;
 }
 
-// Longest-first tiles (lpt_heads), A/B in one process against pairs (bitwise-equal outputs):
-// B64 H6 T256 causal +9%, B16 H8 T512 +29% (two-wave workgroups, every tile resident at once).
-// The split forward, where it applies, beats both (B2 H8 N1024: 0.060 ms split, 0.084 ms
-// longest-first), so a split launch keeps the pairs.
+// Longest-first tiles (lpt_heads) against pairs (bitwise-equal outputs): B8 H8 T512 causal 32.4 and
+// 42.8 us (two-wave workgroups, every tile resident at once).  A split launch keeps the pairs: the
+// split, where it applies, mostly beats both (B2 H8 N1024 D128: 84 us, 109 longest-first).
 
 template <int HS, bool CAUSAL>
 void launch_fwd(const float* q, const float* k, const float* v, float* o, float* l, int nh,

@@ -24,9 +24,9 @@ int gemm_launch(const GemmOperand& A, const GemmOperand& B, const GemmOut& C,
   // 64x128 where 128x128 would leave most CUs one workgroup and some two (2048 x 2304 x 384: 31.8
   // us, 128x128 34.2; 8192 x 576 x 384 32.8 and 34.5) and the loads are the ones whose kernels hold
   // three workgroups a CU (the weight gradient's 64x128 kernel holds two: 1216 x 3456 x 14775 1571
-  // us, 128x128 1030).  Otherwise 128x128 (16384 x 768 x 384: 60 us, 64x128 68; 8192 x 1536 x 384 61 and 68;
-  // 8192 x 384 x 384 23.9 and 25.2).  The tile never depends on the pointwise stage, and all of them
-  // sum in the same order.
+  // us, 128x128 1030).  Otherwise 128x128 (16384 x 768 x 384: 60 us, 64x128 68; 8192 x 1536 x 384
+  // 61 and 68; 8192 x 384 x 384 23.9 and 25.2).  The tile never depends on the pointwise stage, and
+  // all of them sum in the same order.
   const int64_t m64 = (M + 63) / 64 * Z, n128 = (N + 127) / 128;
   const int64_t wide = (M + 127) / 128 * Z * n128;
   if (m64 * n128 < 256 || m64 * ((N + 63) / 64) <= 640)
@@ -194,8 +194,8 @@ extern "C" int64_t cta_linear_weight_bias_grad_workspace(int64_t rows, int64_t k
 }
 
 // dW = x^T dy as one GEMM over the rows (A = x^T through x's strides), with db = the column sums
-// of dy taken from the GEMM's own dy slices when dy is n-contiguous with n % 4 == 0; otherwise
-// the GEMM and then the column-sum kernels.
+// of dy taken from the GEMM's own dy slices when dy is n-contiguous (kVecMN: any n and alignment);
+// otherwise the GEMM and then the column-sum kernels.
 extern "C" int cta_linear_weight_bias_grad(const float* x, const int64_t* x_strides,
                                            const float* dy, const int64_t* dy_strides,
                                            int64_t rows, int64_t k, int64_t n, float* dw,

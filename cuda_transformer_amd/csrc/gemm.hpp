@@ -37,7 +37,7 @@ struct GemmEpilogue {
   int act = kActNone;
   float* aux = nullptr;  // same (batch, m, n) layout as the output; read-only for the *Grad acts and kActMulAux
   // Nullable: receives the column sums of B over K (sum_k B[k][n], n < N).  Needs Z == 1,
-  // B contiguous along n with N % 4 == 0, no pointwise stage and no mask.
+  // B in load mode kVecMN (contiguous along n), no pointwise stage and no mask.
   float* colsum = nullptr;
 };
 

@@ -23,14 +23,14 @@
 // one rounding of the large accumulator per 16 k instead of sixteen the result is closer to the
 // exact product than the FP32 MFMA's (relative error at K = 768, N(0,1) operands: 1.6e-7 against
 // 5.0e-7; K = 8192: 5.7e-7 against 1.6e-6).
-// Sustained on all CUs, from registers, the six products reach 305 TFLOP/s of FP32 work (the
+// Sustained on all CUs, from registers, the six products reach 305-312 TFLOP/s of FP32 work (the
 // chip's power limit), the FP32 MFMA 154.
 // Operands are scaled by 2^24 before the split (split_bf16.hpp), so that the parts hold every float
 // below 2^103 exactly, subnormals included, and products keep their bits down to where FP32's own
 // end.  Sums above 2^79 overflow, infinities and larger operands give NaN: a workgroup whose tile
 // comes out with a value that is not finite discards it and runs the tile again with FP32 MFMAs
-// (exact_tile), so such operands give what FP32 arithmetic gives, in up to 2.4 times the time
-// (8192 x 3072 x 768 with an infinity in every tile: 212 -> 516 us).
+// (exact_tile), so such operands give what FP32 arithmetic gives, in up to 2.7 times the time
+// (8192 x 3072 x 768 with an infinity in every tile: 195-201 -> 528 us).
 //
 // gfx950 design: workgroup tile 128x128 of four 64x64 waves, 64x128 of four 32x64 or 64x64 of
 // four 32x32, two or three workgroups (waves per SIMD) on a CU.  A lane loads eight k of one row
@@ -41,10 +41,9 @@
 // Loads and the epilogue's stores go through buffer resources: scalar bases with fixed per-lane
 // offsets, and the buffer's range check zeroes (loads) or drops (stores) what lies outside the
 // operand, so the K loop and the epilogue carry no per-element address arithmetic or bounds
-// tests.  What bounds it: 8192 x 3072 x 768 runs at 182 TFLOP/s (FP32 MFMA: 142; without the scale
-// 185, with the matrix pipe 54% busy at 1.93 GHz), at the chip's power limit (on all-zero operands
-// the same kernel clocks 2.45 GHz and takes 167 us instead of 209), so bytes moved per product and
-// the splits' instructions cost time too.
+// tests.  What bounds it: 8192 x 3072 x 768 runs at 192-199 TFLOP/s (FP32 MFMA: 142), the matrix
+// pipe 60% busy at 1.77 GHz, at the chip's power limit (on all-zero operands the same kernel takes
+// 142 us instead of 195-201), so bytes moved per product and the splits' instructions cost time too.
 //
 // This header holds the kernel templates and the per-tile launcher; gemm_tiles_*.hip each
 // instantiate a few tile types (gemm_launch_<tile>), so the build compiles them in parallel, and
@@ -111,8 +110,8 @@ __device__ __forceinline__ void unit_coords(int f, int& r, int& h) {
 // of range; kAnyK, whose end may fall inside a lane's four k, loads that slice by single dwords
 // (its whole slices are dwordx4 loads too: buffer loads need only 4-byte alignment).  kStrided
 // loads every slice by single dwords, rows past the end moved out of range, and zeroes k past the
-// end in registers (2048 x 3072 x 768 with every second column of a wider x: 107 us, 132 with
-// kScalar loads of both operands; with every second column of a wider W 70 and 134).
+// end in registers (2048 x 3072 x 768 with every second column of a wider x: 103 us, 132 with
+// kScalar loads of both operands; with every second column of a wider W 69 and 134).
 template <int MODE, int ROWS, int THREADS>
 struct LoadPlan {
   using S = Slice<ROWS, THREADS>;

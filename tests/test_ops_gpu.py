@@ -414,10 +414,9 @@ def test_db_strided_views(cuda):
     assert torch.equal(db_calculation(big), db_calculation(big))
 
 
-# (rows, k, n): split-K with the SplitTile (GPT qkv / fc2 weight gradients, config 4), one
-# unsplit 128x128-tile GEMM (256 tiles), unsplit narrow tiles with ragged rows, the unsplit
-# 192-column tiles (64x192 with K-slices of 16 and 32, 128x192), and n % 4 != 0 (dy not
-# vector-loadable: GEMM then the column-sum kernels).
+# (rows, k, n): split-K (GPT qkv / fc2 weight gradients, config 4), one unsplit 128x128-tile GEMM
+# (256 tiles), small outputs with ragged rows, k and n, and an odd n.  dy is contiguous in all of
+# them, so db comes out of the GEMM; the column-sum route is test_weight_bias_grad_column_strides.
 WB_SHAPES = [(16384, 384, 1152), (16384, 1536, 384), (8192, 768, 3072), (2048, 2048, 2048),
              (333, 64, 100), (1000, 20, 36), (300, 64, 192), (800, 128, 384), (1000, 256, 1152),
              (100, 48, 65), (5, 7, 12)]
